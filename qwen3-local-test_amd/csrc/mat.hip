@@ -3,18 +3,21 @@
 //
 // Replaces Qwen4Vulkan::mat (src/qwen4_vk.cpp:848-856) on its matrix-vector pipelines q4_matmul_q8 /
 // q4_matmul_f32 (shaders/q4_matmul.comp with the C_Q8 / C_F32 codecs of shaders/q4_codec.glsl; the planar
-// repacking of GGUF Q8_0 is src/qwen4_vk.cpp:98-106) below 16 tokens, and on its tiled GEMM pipelines
-// q4_gemm_q8 / q4_gemm_f32 from 16 (further down: a skinny MFMA kernel for Q8 up to 64 tokens, a tiled
-// MFMA GEMM beyond): every output is the fp32 dot product of a dequantized
-// weight row (int8 times its block's scale) with a token's input row, then optionally silu(y * post_scale).
+// repacking of GGUF Q8_0 is src/qwen4_vk.cpp:98-106) and on its tiled GEMM pipelines q4_gemm_q8 / q4_gemm_f32:
+// every output is the fp32 dot product of a dequantized weight row (int8 times its block's scale) with a
+// token's input row, then optionally silu(y * post_scale). One token, and fp32 weights below 16: matrix-vector
+// kernels. Q8 from two tokens to a few hundred: the token-tile MFMA kernel. Beyond, and fp32 weights from 16:
+// the tiled MFMA GEMM.
 //
 // MI355X design of the matrix-vector kernels: the weights are read once per launch and are the bound (a
-// decode step's projections are memory-bound); a wave owns RW rows and a workgroup NTP tokens (one for a single token), lane l covering the
-// 16 consecutive columns 16 l + 1,024 k of every row, so a wave reads a kilobyte of each row per chunk in
-// one 16-byte load a lane (plus one scale a lane pair), and every weight load of a wave's rows is issued
-// before the first is used. A 16-column group never crosses a 32-weight block, so the lane applies its
-// block scale once per group and token. The partial dot products are summed over the wave with DPP row
-// operations and permlane swaps.
+// decode step's projections are memory-bound); a wave owns RW rows and a workgroup one token (f32: up to four),
+// lane l covering the 16 consecutive columns 16 l + 1,024 k of every row, so a wave reads a kilobyte of each row
+// per chunk in one 16-byte load a lane (plus one scale a lane pair), and every weight load of a wave's rows is
+// issued before the first is used. A 16-column group never crosses a 32-weight block, so the lane applies its
+// block scale once per group. The partial dot products are summed over the wave with DPP row operations and
+// permlane swaps.
+#include <atomic>
+
 #include "common.hpp"
 #include "kernels.hpp"
 
@@ -22,7 +25,12 @@ namespace qw {
 
 namespace {
 
-constexpr int kMatNTP = 4;  // tokens a workgroup
+typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
+
+constexpr int kMatNTP = 4;  // tokens a workgroup (f32 weights)
 
 // Sum over the 64 lanes, in every lane.
 __device__ __forceinline__ float mat_wave_sum(float x) {
@@ -88,21 +96,17 @@ __device__ __forceinline__ void mat_f32_body(const MatArgs& a, int bx) {
 // matrix in flight at once (the stream is the bound: the loads have to overlap); then per chunk the token
 // rows' 16 columns (cached: every wave reads them) and the dot products
 constexpr int kMatK = 4;
-template <int NTP, int RW>
+template <int RW>
 __device__ __forceinline__ void mat_q8_body(const MatArgs& a, int bx) {
-    typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
     const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
     const int r0 = (bx * 4 + wave) * RW;
-    const int t0 = blockIdx.y * NTP;
-    const int nt = min(NTP, a.n - t0);
+    const int t = blockIdx.y;
     if (r0 >= a.rows) return;  // whole waves
     const int8_t* w8 = static_cast<const int8_t*>(a.w);
     const int nsb = a.cols >> 5;  // scales a row
-    float acc[RW][NTP];
+    float acc[RW];
 #pragma unroll
-    for (int r = 0; r < RW; r++)
-#pragma unroll
-        for (int t = 0; t < NTP; t++) acc[r][t] = 0.f;
+    for (int r = 0; r < RW; r++) acc[r] = 0.f;
     for (int cb = 0; cb < a.cols; cb += kMatK * 1024) {
         u32x4 q[RW][kMatK];
         float sc[RW][kMatK];
@@ -122,15 +126,12 @@ __device__ __forceinline__ void mat_q8_body(const MatArgs& a, int bx) {
             if (cb + k * 1024 >= a.cols) break;
             const int c = cb + k * 1024 + lane * 16;
             if (c >= a.cols) continue;  // this lane's group lies past the row
-            float xv[NTP][16];
+            float xv[16];
+            const float* xr = a.x + (size_t)t * a.x_stride + c;
 #pragma unroll
-            for (int t = 0; t < NTP; t++) {
-                const float* xr = a.x + (size_t)(t0 + (t < nt ? t : 0)) * a.x_stride + c;
-#pragma unroll
-                for (int i = 0; i < 16; i += 4) {
-                    const f32x4 v = *reinterpret_cast<const f32x4*>(xr + i);
-                    xv[t][i] = v[0], xv[t][i + 1] = v[1], xv[t][i + 2] = v[2], xv[t][i + 3] = v[3];
-                }
+            for (int i = 0; i < 16; i += 4) {
+                const f32x4 v = *reinterpret_cast<const f32x4*>(xr + i);
+                xv[i] = v[0], xv[i + 1] = v[1], xv[i + 2] = v[2], xv[i + 3] = v[3];
             }
 #pragma unroll
             for (int r = 0; r < RW; r++) {
@@ -143,32 +144,27 @@ __device__ __forceinline__ void mat_q8_body(const MatArgs& a, int bx) {
                     wv[4 * j + 2] = (float)((v << 8) >> 24);
                     wv[4 * j + 3] = (float)(v >> 24);
                 }
+                float d = 0.f;
 #pragma unroll
-                for (int t = 0; t < NTP; t++) {
-                    float d = 0.f;
-#pragma unroll
-                    for (int i = 0; i < 16; i++) d = __builtin_fmaf(wv[i], xv[t][i], d);
-                    acc[r][t] = __builtin_fmaf(d, sc[r][k], acc[r][t]);
-                }
+                for (int i = 0; i < 16; i++) d = __builtin_fmaf(wv[i], xv[i], d);
+                acc[r] = __builtin_fmaf(d, sc[r][k], acc[r]);
             }
         }
     }
 #pragma unroll
-    for (int r = 0; r < RW; r++)
-#pragma unroll
-        for (int t = 0; t < NTP; t++) {
-            float v = mat_wave_sum(acc[r][t]);
-            if (a.post == 1) {
-                const float u = v * a.post_scale;
-                v = u / (1.0f + __expf(-u));
-            }
-            if (lane == 0 && r0 + r < a.rows && t < nt) a.y[(size_t)(t0 + t) * a.y_stride + r0 + r] = v;
+    for (int r = 0; r < RW; r++) {
+        float v = mat_wave_sum(acc[r]);
+        if (a.post == 1) {
+            const float u = v * a.post_scale;
+            v = u / (1.0f + __expf(-u));
         }
+        if (lane == 0 && r0 + r < a.rows) a.y[(size_t)t * a.y_stride + r0 + r] = v;
+    }
 }
 
-template <int NTP, int RW>
+template <int RW>
 __global__ __launch_bounds__(256) void k_mat_q8(MatArgs a) {
-    mat_q8_body<NTP, RW>(a, blockIdx.x);
+    mat_q8_body<RW>(a, blockIdx.x);
 }
 template <int NTP, int RW>
 __global__ __launch_bounds__(256) void k_mat_f32(MatArgs a) {
@@ -182,7 +178,7 @@ __global__ __launch_bounds__(256) void k_mat_multi(MatMultiArgs a) {
     int i = 0;
     while (i + 1 < a.count && (int)blockIdx.x >= a.wg_end[i]) i++;
     const int bx = (int)blockIdx.x - (i ? a.wg_end[i - 1] : 0);
-    if constexpr (Q8) mat_q8_body<NTP, RW>(a.m[i], bx);
+    if constexpr (Q8) mat_q8_body<RW>(a.m[i], bx);
     else mat_f32_body<NTP, RW>(a.m[i], bx);
 }
 
@@ -199,8 +195,6 @@ __global__ __launch_bounds__(256) void k_mat_multi(MatMultiArgs a) {
 // lo.hi, lo.lo). The next step's global loads are in flight while the current step's MFMAs run; tiles are
 // assigned so that each XCD takes a contiguous range of row tiles (its weights stay in its L2).
 constexpr int kGemmBM = 128;  // rows a workgroup
-typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
-typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 
 // Byte offset of 16-byte chunk g (k = 8 g .. 8 g + 7) of tile row r in an LDS tile of [rows][32] bf16: the
 // chunk index is XORed with (r / 2) % 4, so any 8 consecutive rows' chunk g (an MFMA operand read) and any
@@ -216,116 +210,265 @@ __device__ __forceinline__ void split_bf16(const float (&v)[8], bf16x8& hi, bf16
     }
 }
 
-// ---- a few tokens (16 to a few hundred), Q8: skinny MFMA kernel ------------------------------------
-// The tiled GEMM keeps too little in flight there (its 128-row tiles give the 8,192-row projection only 64
-// workgroups below 32 tokens). Here a workgroup owns 32 rows x 16 tokens and its four waves split the
-// columns; a wave loads its weights straight from HBM in the MFMA operand layout (lane (c, g): row c, the
-// 8 columns 8 g .. 8 g + 7 of a 32-column block, one 8-byte load), kSkK blocks at a time, all issued before
-// the first is used, with the token rows (fp32, split into bf16 hi / lo as in the GEMM) and the block
-// scales of its accumulator rows. Per block and 16-row tile: two MFMAs (hi, lo) into a fresh accumulator,
-// scaled into the running sum. The four waves' sums meet in LDS.
-constexpr int kSkinnyMaxN = 64;  // token counts the skinny kernel takes (from 16)
-constexpr int kSkinnyMaxRows = 1024;         // row counts it takes at any token count
-// TT 16-token tiles a workgroup, KK blocks a batch
-template <int TT, int KK>
-__global__ __launch_bounds__(256) void k_mat_skinny(MatArgs a) {
-    typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
-    __shared__ f32x4 s_acc[3][2][TT][64];
-    const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, c = lane & 15, g = lane >> 4;
-    const int r0 = blockIdx.x * 32, t0 = blockIdx.y * 16 * TT;
-    const int nkb = a.cols >> 5;
-    const int kb0 = wave * nkb / 4, kb1 = (wave + 1) * nkb / 4;  // this wave's blocks
-    const int8_t* w8 = static_cast<const int8_t*>(a.w);
-    const size_t arow[2] = {(size_t)min(r0 + c, a.rows - 1) * a.cols, (size_t)min(r0 + 16 + c, a.rows - 1) * a.cols};
-    int srow[2][4];  // accumulator rows of this lane: 16 m + 4 g + i
+// ---- two to a few hundred tokens, Q8: token-tile MFMA kernel, the columns split over the waves -----------
+// A workgroup owns 16 R rows x 16 TT tokens and its waves split the columns: wave w takes the 128-column quads
+// w, w + KW, ... (four Q8 blocks each), so that nothing is loaded or converted twice in a workgroup and no
+// barrier is needed before the waves' sums meet. Weights are the B operand: an accumulator column is then a
+// weight row, its block scale one value a lane.
+//
+// What bounds it is the rate of the vector-memory pipe and of instruction issue, not HBM. A load costs one cycle
+// per 64-byte piece it touches, so an operand loaded straight in the MFMA layout (lane l: row l % 16) costs 64
+// cycles a kilobyte; loaded by consecutive lanes it costs 16, and a pass through the wave's own part of the LDS
+// (written as loaded, read as operands, both free of bank conflicts by the XORs below; in-order within the
+// wave) gives the layout. 9,216 x 2,048 at 4 / 77 tokens, one box: 10.9 / 31.1 us with operand-layout loads,
+// 8.5 / 20.7 us through the LDS; the kernels before (fp32 multiply-adds on up to 4 tokens a workgroup; 32-row
+// workgroups with operand-layout loads from 16) took 16.0 / 86 us. A vector instruction, the conversions
+// included, takes a SIMD 2.0-2.5 ns.
+//
+// fp32 accuracy from bf16 products: an int8 weight is exact in bf16; NS = 2 splits x into hi + lo (up to 2^-18 of
+// |x| left, 2.5e-6 in an output), NS = 3 into three parts (2^-27 left: 1.1e-7, the level of fp32 sums), for the
+// token counts below 16.
+__device__ __forceinline__ uint32_t pk_bf16(float a, float b) {  // one v_cvt_pk_bf16_f32
+    return __builtin_bit_cast(uint32_t, __builtin_convertvector(f32x2{a, b}, bf16x2));
+}
+
+// Eight int8 weights (two words) as bf16, exactly.
+__device__ __forceinline__ bf16x8 weights_bf16(uint32_t lo, uint32_t hi) {
+    u32x4 w;
 #pragma unroll
-    for (int m = 0; m < 2; m++)
-#pragma unroll
-        for (int i = 0; i < 4; i++) srow[m][i] = min(r0 + 16 * m + 4 * g + i, a.rows - 1);
-    const float* xrow[TT];
-#pragma unroll
-    for (int t = 0; t < TT; t++) xrow[t] = a.x + (size_t)min(t0 + 16 * t + c, a.n - 1) * a.x_stride + 8 * g;
-    f32x4 acc[2][TT];
-#pragma unroll
-    for (int m = 0; m < 2; m++)
-#pragma unroll
-        for (int t = 0; t < TT; t++) acc[m][t] = f32x4{0.f, 0.f, 0.f, 0.f};
-    for (int kb = kb0; kb < kb1; kb += KK) {
-        u32x2 wq[2][KK];
-        f32x4 xv[KK][TT][2];
-        float sc[2][4][KK];
-#pragma unroll
-        for (int j = 0; j < KK; j++) {
-            const int b = min(kb + j, kb1 - 1);  // past this wave's range: a repeat, unused
-#pragma unroll
-            for (int m = 0; m < 2; m++) wq[m][j] = *reinterpret_cast<const u32x2*>(w8 + arow[m] + b * 32 + 8 * g);
-#pragma unroll
-            for (int t = 0; t < TT; t++) {
-                xv[j][t][0] = *reinterpret_cast<const f32x4*>(xrow[t] + b * 32);
-                xv[j][t][1] = *reinterpret_cast<const f32x4*>(xrow[t] + b * 32 + 4);
-            }
-#pragma unroll
-            for (int m = 0; m < 2; m++)
-#pragma unroll
-                for (int i = 0; i < 4; i++) sc[m][i][j] = a.s[(size_t)srow[m][i] * nkb + b];
-        }
-#pragma unroll
-        for (int j = 0; j < KK; j++) {
-            if (kb + j >= kb1) break;  // uniform
-            bf16x8 av[2];
-#pragma unroll
-            for (int m = 0; m < 2; m++)
-#pragma unroll
-                for (int e = 0; e < 8; e++) {
-                    const int q = (int)wq[m][j][e / 4];
-                    av[m][e] = (__bf16)(float)((q << (24 - 8 * (e % 4))) >> 24);
-                }
-#pragma unroll
-            for (int t = 0; t < TT; t++) {
-                float v8[8] = {xv[j][t][0][0], xv[j][t][0][1], xv[j][t][0][2], xv[j][t][0][3],
-                               xv[j][t][1][0], xv[j][t][1][1], xv[j][t][1][2], xv[j][t][1][3]};
-                bf16x8 bh, bl;
-                split_bf16(v8, bh, bl);
-#pragma unroll
-                for (int m = 0; m < 2; m++) {
-                    f32x4 p = __builtin_amdgcn_mfma_f32_16x16x32_bf16(av[m], bh, f32x4{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
-                    p = __builtin_amdgcn_mfma_f32_16x16x32_bf16(av[m], bl, p, 0, 0, 0);
-#pragma unroll
-                    for (int i = 0; i < 4; i++) acc[m][t][i] = __builtin_fmaf(sc[m][i][j], p[i], acc[m][t][i]);
-                }
-            }
-        }
+    for (int e = 0; e < 4; e++) {
+        const int v = (int)(e < 2 ? lo : hi), s = 16 * (e & 1);
+        w[e] = pk_bf16((float)((v << (24 - s)) >> 24), (float)((v << (16 - s)) >> 24));
     }
-    // the four waves' column ranges: sum in LDS, wave 0 writes (lane (c, g): token 16 t + c, rows 16 m + 4 g + i)
-    if (wave > 0) {
+    return __builtin_bit_cast(bf16x8, w);
+}
+
+// KW waves; B > 1 (TT = 1, up to 16 / B tokens): B consecutive blocks share the rows of one A operand, block j
+// of them in rows [16 j / B, 16 (j + 1) / B), so that their token values are split in one go; a block's product
+// is then valid in the lanes of its rows only, which take it with their own block's scale.
+template <int TT, int R, int NS, int B>
+struct TokLds {  // a wave's part of the LDS
+    unsigned char w[R][2048];       // a quad of 16 rows: [row][8 chunks of 16 columns], chunk ^ (row / 2) % 8
+    float s[R][64];                 // their scales [row][block]
+    unsigned char x[TT][NS][1024];  // an A operand's parts: [8-column group][row ^ 4 group], 16 bytes
+};
+
+template <int TT, int R, int NS, int B, int KW>
+__device__ __forceinline__ void mat_tok_body(const MatArgs& a, int bx, int by, unsigned char* smem) {
+    static_assert(B == 1 || TT == 1, "shared rows: one token tile");
+    typedef TokLds<TT, R, NS, B> Lds;
+    constexpr int U = 4 / B;                        // A operands a quad
+    constexpr int XR = U == 4 && TT >= 3 ? 2 : U;   // token-row buffers: A operands in flight
+    const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
+    const int c = lane & 15, g = lane >> 4;
+    const int r0 = bx * 16 * R, t0 = by * 16 * TT;
+    const int nkb = a.cols >> 5, nq = (nkb + 3) >> 2;
+    constexpr size_t kLds = sizeof(Lds) > R * TT * 1024 ? sizeof(Lds) : R * TT * 1024;  // (the final sums reuse it)
+    Lds& L = *reinterpret_cast<Lds*>(smem + wave * kLds);
+    // rows past the matrix, tokens past the last and columns past the row (kFar added) lie outside the
+    // resources: such loads read zero and cause no traffic, so no load is conditional
+    constexpr unsigned kFar = 0x60000000u;
+    const int nr = min(16 * R, a.rows - r0), nt = min(16 * TT, a.n - t0);
+    const __amdgpu_buffer_rsrc_t rw = __builtin_amdgcn_make_buffer_rsrc(
+        const_cast<int8_t*>(static_cast<const int8_t*>(a.w)) + (size_t)r0 * a.cols, (short)0, nr * a.cols, 0x00020000);
+    const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc(
+        const_cast<float*>(a.s) + (size_t)r0 * nkb, (short)0, nr * nkb * 4, 0x00020000);
+    const __amdgpu_buffer_rsrc_t rx = __builtin_amdgcn_make_buffer_rsrc(
+        const_cast<float*>(a.x) + (size_t)t0 * a.x_stride, (short)0, ((nt - 1) * a.x_stride + a.cols) * 4, 0x00020000);
+
+    // loads: 16 bytes a lane, whole cache lines by consecutive lanes. Weights: load i of a quad is rows
+    // 8 i + lane / 8, chunk lane % 8. Scales: row lane / 4, block lane % 4. Token rows: load i of an A operand is
+    // piece 64 i + lane of its [16 / B tokens][32 B columns].
+    u32x4 wq[R][2];
+    float sq[R];
+    f32x4 xv[XR][TT][2];
+    auto load_w = [&](int q) {
+        const int col = 128 * q + 16 * (lane & 7), blk = 4 * q + (lane & 3);
+        const unsigned cw = col < a.cols ? (unsigned)col : kFar, cs = blk < nkb ? 4u * blk : kFar;
 #pragma unroll
-        for (int m = 0; m < 2; m++)
+        for (int r = 0; r < R; r++) {
 #pragma unroll
-            for (int t = 0; t < TT; t++) s_acc[wave - 1][m][t][lane] = acc[m][t];
+            for (int i = 0; i < 2; i++)
+                wq[r][i] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(
+                    rw, (int)((16 * r + 8 * i + (lane >> 3)) * a.cols + cw), 0, 0));
+            sq[r] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(rs, (int)((16 * r + (lane >> 2)) * nkb * 4 + cs), 0, 0));
+        }
+    };
+    int xoff[TT][2];  // the pieces' token rows
+#pragma unroll
+    for (int t = 0; t < TT; t++)
+#pragma unroll
+        for (int i = 0; i < 2; i++) {
+            const int p = 64 * i + lane, tok = 16 * t + p / (8 * B);
+            xoff[t][i] = tok < nt ? (tok * a.x_stride + 4 * (p % (8 * B))) * 4 : (int)kFar;
+        }
+    const int xblk = (lane % (8 * B)) / 8;  // this lane's block of the A operand
+    auto load_x = [&](auto k_, int b) {
+        constexpr int k = k_;
+        const unsigned o = b + xblk < nkb ? 128u * b : kFar;
+#pragma unroll
+        for (int t = 0; t < TT; t++)
+#pragma unroll
+            for (int i = 0; i < 2; i++)
+                xv[k][t][i] = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(rx, (int)(xoff[t][i] + o), 0, 0));
+    };
+    // LDS places: of this lane's pieces (written) and fragments (read)
+    int wst[2], xst[2], wld[4];
+#pragma unroll
+    for (int i = 0; i < 2; i++) {
+        const int row = 8 * i + (lane >> 3);
+        wst[i] = row * 128 + (((lane & 7) ^ ((row >> 1) & 7)) << 4);
+        const int p = 64 * i + lane, xr = (p % (8 * B)) / 8 * (16 / B) + p / (8 * B), pc = p % 8;
+        xst[i] = ((pc >> 1) * 16 + (xr ^ ((pc >> 1) << 2))) * 16 + (pc & 1) * 8;
     }
-    __syncthreads();
-    if (wave == 0) {
 #pragma unroll
-        for (int t = 0; t < TT; t++) {
-            const int tok = t0 + 16 * t + c;
+    for (int j = 0; j < 4; j++) wld[j] = c * 128 + (((2 * j + (g >> 1)) ^ ((c >> 1) & 7)) << 4) + (g & 1) * 8;
+    const int xld = (g * 16 + (c ^ (g << 2))) * 16;
+
+    f32x4 acc[R][TT];
 #pragma unroll
-            for (int m = 0; m < 2; m++) {
-                f32x4 v = acc[m][t];
+    for (int r = 0; r < R; r++)
 #pragma unroll
-                for (int w = 0; w < 3; w++) v += s_acc[w][m][t][lane];  // waves 1..3 in order
+        for (int t = 0; t < TT; t++) acc[r][t] = f32x4{0.f, 0.f, 0.f, 0.f};
+    // first block of the j-th A operand from quad q on
+    auto block_of = [&](int q, int j) { return 4 * (q + KW * (j / U)) + B * (j % U); };
+    load_w(wave);
+    static_for<0, XR>([&](auto j) { load_x(j, block_of(wave, j)); });
+#pragma unroll 1
+    for (int q = wave; q < nq; q += KW) {
 #pragma unroll
-                for (int i = 0; i < 4; i++) {
-                    const int row = r0 + 16 * m + 4 * g + i;
-                    float y = v[i];
-                    if (a.post == 1) {
-                        const float u = y * a.post_scale;
-                        y = u / (1.0f + __expf(-u));
+        for (int r = 0; r < R; r++) {
+#pragma unroll
+            for (int i = 0; i < 2; i++) *reinterpret_cast<u32x4*>(L.w[r] + wst[i]) = wq[r][i];
+            L.s[r][lane] = sq[r];
+        }
+        load_w(q + KW);
+        float sc[R][U];
+#pragma unroll
+        for (int r = 0; r < R; r++)
+#pragma unroll
+            for (int u = 0; u < U; u++) sc[r][u] = L.s[r][4 * c + (B == 1 ? u : B == 2 ? 2 * u + (g >> 1) : g)];
+        static_for<0, U>([&](auto u_) {
+            constexpr int u = u_, xb = u % XR;
+            // the A operand's token values: split and laid out
+#pragma unroll
+            for (int t = 0; t < TT; t++)
+#pragma unroll
+                for (int i = 0; i < 2; i++) {
+                    uint32_t part[NS][2];
+#pragma unroll
+                    for (int e = 0; e < 2; e++) {
+                        float v0 = xv[xb][t][i][2 * e], v1 = xv[xb][t][i][2 * e + 1];
+#pragma unroll
+                        for (int k = 0; k < NS; k++) {
+                            const uint32_t w = pk_bf16(v0, v1);
+                            part[k][e] = w;
+                            if (k + 1 < NS) {
+                                const float h0 = __uint_as_float(w << 16), h1 = __uint_as_float(w & 0xFFFF0000u);
+                                // three parts: an infinity is its first part (as fp32 products would have it)
+                                v0 = NS == 3 && k == 0 && __builtin_fabsf(h0) == __builtin_inff() ? 0.f : v0 - h0;
+                                v1 = NS == 3 && k == 0 && __builtin_fabsf(h1) == __builtin_inff() ? 0.f : v1 - h1;
+                            }
+                        }
                     }
-                    if (tok < a.n && row < a.rows) a.y[(size_t)tok * a.y_stride + row] = y;
+#pragma unroll
+                    for (int k = 0; k < NS; k++)
+                        *reinterpret_cast<u32x2*>(L.x[t][k] + xst[i]) = u32x2{part[k][0], part[k][1]};
                 }
+            load_x(std::integral_constant<int, xb>{}, block_of(q, u + XR));
+            if (block_of(q, u) < nkb) {  // uniform; a group's blocks past the row hold zeros
+                f32x4 p[R][TT];
+#pragma unroll
+                for (int jj = 0; jj < B; jj++) {
+                    bf16x8 wv[R];
+#pragma unroll
+                    for (int r = 0; r < R; r++) {
+                        const u32x2 w = *reinterpret_cast<const u32x2*>(L.w[r] + wld[u * B + jj]);
+                        wv[r] = weights_bf16(w[0], w[1]);
+                    }
+#pragma unroll
+                    for (int t = 0; t < TT; t++) {
+                        f32x4 d[R];
+#pragma unroll
+                        for (int k = 0; k < NS; k++) {
+                            const bf16x8 part = *reinterpret_cast<const bf16x8*>(L.x[t][k] + xld);
+#pragma unroll
+                            for (int r = 0; r < R; r++)
+                                d[r] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(part, wv[r], k ? d[r] : f32x4{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
+                        }
+#pragma unroll
+                        for (int r = 0; r < R; r++) {
+                            if (jj == 0) p[r][t] = d[r];
+                            else
+#pragma unroll
+                                for (int i = 0; i < 4; i++) p[r][t][i] = (g * B) / 4 == jj ? d[r][i] : p[r][t][i];
+                        }
+                    }
+                }
+#pragma unroll
+                for (int t = 0; t < TT; t++)
+#pragma unroll
+                    for (int r = 0; r < R; r++)
+#pragma unroll
+                        for (int i = 0; i < 4; i++) acc[r][t][i] = __builtin_fmaf(sc[r][u], p[r][t][i], acc[r][t][i]);
             }
+        });
+    }
+    // shared rows: the groups of lanes hold the sums of different blocks
+    if constexpr (B > 1) {
+#pragma unroll
+        for (int r = 0; r < R; r++)
+#pragma unroll
+            for (int i = 0; i < 4; i++) {
+                uint32_t v = __float_as_uint(acc[r][0][i]);
+                const auto h = __builtin_amdgcn_permlane32_swap(v, v, false, false);
+                float f = __uint_as_float(h[0]) + __uint_as_float(h[1]);
+                if constexpr (B == 4) {
+                    v = __float_as_uint(f);
+                    const auto l = __builtin_amdgcn_permlane16_swap(v, v, false, false);
+                    f = __uint_as_float(l[0]) + __uint_as_float(l[1]);
+                }
+                acc[r][0][i] = f;
+            }
+    }
+    // the waves' column ranges meet in LDS (each wave's sums in its own part, read by it alone until here),
+    // summed in wave order; wave w stores tiles w, w + KW, ... (lane (c, g): row 16 r + c, tokens 16 t + 4 g .. + 3)
+#pragma unroll
+    for (int r = 0; r < R; r++)
+#pragma unroll
+        for (int t = 0; t < TT; t++)
+            *reinterpret_cast<f32x4*>(smem + wave * kLds + (r * TT + t) * 1024 + lane * 16) = acc[r][t];
+    __syncthreads();
+    for (int i = wave; i < R * TT; i += KW) {
+        f32x4 v = *reinterpret_cast<const f32x4*>(smem + i * 1024 + lane * 16);
+#pragma unroll
+        for (int w = 1; w < KW; w++) v += *reinterpret_cast<const f32x4*>(smem + w * kLds + i * 1024 + lane * 16);
+        const int row = r0 + 16 * (i / TT) + c, tok = t0 + 16 * (i % TT) + 4 * g;
+        if (row >= a.rows) continue;
+#pragma unroll
+        for (int e = 0; e < 4; e++) {
+            float y = v[e];
+            if (a.post == 1) {
+                const float u = y * a.post_scale;
+                y = u / (1.0f + __expf(-u));
+            }
+            if (tok + e < a.n) a.y[(size_t)(tok + e) * a.y_stride + row] = y;
         }
     }
+}
+
+template <int TT, int R, int NS, int B, int KW>
+constexpr size_t tok_lds() {
+    return KW * (sizeof(TokLds<TT, R, NS, B>) > R * TT * 1024 ? sizeof(TokLds<TT, R, NS, B>) : R * TT * 1024);
+}
+
+// Grid (row groups of every matrix in turn, token groups)
+template <int TT, int R, int NS, int B, int KW>
+__global__ __launch_bounds__(64 * KW) void k_mat_tok(MatMultiArgs a) {
+    extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
+    int i = 0;
+    while (i + 1 < a.count && (int)blockIdx.x >= a.wg_end[i]) i++;
+    mat_tok_body<TT, R, NS, B, KW>(a.m[i], (int)blockIdx.x - (i ? a.wg_end[i - 1] : 0), blockIdx.y, smem);
 }
 
 template <bool Q8, int BN>
@@ -503,20 +646,104 @@ __global__ __launch_bounds__(256, 2) void k_gemm(MatArgs a) {
 
 }  // namespace
 
+namespace {
+
+template <int TT, int R, int NS, int B, int KW>
+hipError_t launch_tok(MatMultiArgs a, hipStream_t s) {
+    constexpr size_t lds = tok_lds<TT, R, NS, B, KW>();
+    if constexpr (lds > 64 * 1024) {  // past the default limit: raised once per device
+        static std::atomic<uint64_t> raised{0};
+        int dev = 0;
+        if (hipGetDevice(&dev) != hipSuccess) return hipErrorInvalidDevice;
+        const uint64_t bit = 1ull << (dev & 63);
+        if (!(raised.load(std::memory_order_acquire) & bit)) {
+            const hipError_t e = hipFuncSetAttribute((const void*)k_mat_tok<TT, R, NS, B, KW>,
+                                                     hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+            if (e != hipSuccess) return e;
+            raised.fetch_or(bit, std::memory_order_acq_rel);
+        }
+    }
+    int wg = 0;
+    for (int i = 0; i < a.count; i++) a.wg_end[i] = wg += (a.m[i].rows + 16 * R - 1) / (16 * R);
+    hipLaunchKernelGGL((k_mat_tok<TT, R, NS, B, KW>), dim3(wg, (a.m[0].n + 16 * TT - 1) / (16 * TT)), dim3(64 * KW), lds, s, a);
+    return hipGetLastError();
+}
+
+// The token-tile kernel's shapes with two parts a token value. Eight waves (a workgroup a CU) up to 64 tokens, or
+// from 4,096 columns; four (two workgroups a CU) otherwise: 9,216 x 2,048 at 64 / 80 / 256 tokens 16.6 / 23.7 /
+// 56 us with eight, 18.9 / 20.5 / 46 with four; 2,048 x 4,096 at 80 / 256 14.2 / 20.6 and 16.0 / 23.9. The wave
+// count decides the order of a sum, so it depends on nothing that differs between qwattn_mat and
+// qwattn_mat_multi; the tile counts do not.
+struct TokShape {
+    int tt, r;
+    hipError_t (*launch)(MatMultiArgs, hipStream_t);
+};
+constexpr TokShape kTok8[] = {{1, 1, launch_tok<1, 1, 2, 1, 8>}, {1, 2, launch_tok<1, 2, 2, 1, 8>},
+                              {1, 3, launch_tok<1, 3, 2, 1, 8>}, {1, 4, launch_tok<1, 4, 2, 1, 8>},
+                              {2, 2, launch_tok<2, 2, 2, 1, 8>}, {2, 3, launch_tok<2, 3, 2, 1, 8>},
+                              {2, 4, launch_tok<2, 4, 2, 1, 8>}, {3, 2, launch_tok<3, 2, 2, 1, 8>},
+                              {3, 3, launch_tok<3, 3, 2, 1, 8>}, {3, 4, launch_tok<3, 4, 2, 1, 8>},
+                              {4, 3, launch_tok<4, 3, 2, 1, 8>}};
+constexpr TokShape kTok4[] = {{1, 2, launch_tok<1, 2, 2, 1, 4>}, {1, 4, launch_tok<1, 4, 2, 1, 4>},
+                              {2, 4, launch_tok<2, 4, 2, 1, 4>}};
+constexpr int kCus = 256;
+
+// Whether a Q8 matrix takes the token-tile kernel (from two tokens): up to 512 tokens, at any count for matrices
+// of up to 1,024 rows, and wherever the GEMM would have fewer than 256 tiles of 128 rows x 32 tokens.
+bool tok_wins(int rows, int n) {
+    return n <= 512 || rows <= 1024 || ((rows + kGemmBM - 1) / kGemmBM) * ((n + 31) / 32) < 256;
+}
+
+// Row groups of 16 R rows, every matrix by itself.
+int row_groups(const MatMultiArgs& a, int r) {
+    int g = 0;
+    for (int i = 0; i < a.count; i++) g += (a.m[i].rows + 16 * r - 1) / (16 * r);
+    return g;
+}
+
+// Whether the token-tile kernel's 32-bit offsets reach every operand (up to 64 rows and tokens a workgroup).
+bool tok_fits(const MatMultiArgs& a) {
+    const MatArgs& m = a.m[0];
+    return m.cols <= 1 << 24 && (63ll * m.x_stride + m.cols) * 4 < 0x60000000ll;
+}
+
+hipError_t launch_tok_any(const MatMultiArgs& a, hipStream_t s) {
+    const MatArgs& m = a.m[0];
+    if (m.n < 16) {
+        // as many row tiles a workgroup as leave a workgroup a CU, three at most (9,216 x 2,048 at 12 tokens: one
+        // tile 13.1 us, two 12.2, three 9.9, four 11.2)
+        const int r = row_groups(a, 1) <= kCus ? 1 : row_groups(a, 2) <= kCus ? 2 : 3;
+        if (m.n <= 4)
+            return r == 1 ? launch_tok<1, 1, 3, 4, 8>(a, s) : r == 2 ? launch_tok<1, 2, 3, 4, 8>(a, s) : launch_tok<1, 3, 3, 4, 8>(a, s);
+        if (m.n <= 8)
+            return r == 1 ? launch_tok<1, 1, 3, 2, 8>(a, s) : r == 2 ? launch_tok<1, 2, 3, 2, 8>(a, s) : launch_tok<1, 3, 3, 2, 8>(a, s);
+        return r == 1 ? launch_tok<1, 1, 3, 1, 8>(a, s) : r == 2 ? launch_tok<1, 2, 3, 1, 8>(a, s) : launch_tok<1, 3, 3, 1, 8>(a, s);
+    }
+    const int tiles = (m.n + 15) / 16;
+    const auto wgs = [&](const TokShape& k) { return row_groups(a, k.r) * ((tiles + k.tt - 1) / k.tt); };
+    if (m.n <= 64 || m.cols >= 4096) {
+        // instructions a block: splitting and laying out a token tile, converting a row tile, the product of both
+        const TokShape* best = nullptr;
+        long long least = 0;
+        for (const TokShape& k : kTok8) {
+            const long long t = (long long)((wgs(k) + kCus - 1) / kCus) * (30 * k.tt + 14 * k.r + 8 * k.tt * k.r);
+            if (!best || t < least) best = &k, least = t;
+        }
+        return best->launch(a, s);
+    }
+    // the largest shape that still gives every CU a workgroup
+    const TokShape* k = &kTok4[2];
+    while (k > kTok4 && wgs(*k) < kCus) k--;
+    return k->launch(a, s);
+}
+
+}  // namespace
+
 hipError_t launch_mat(const MatArgs& a, bool q8, hipStream_t s) {
-    // the skinny kernel up to 64 tokens, at any token count for matrices of up to 1,024 rows, and wherever
-    // the GEMM would have fewer than 256 tiles of 128 rows x 32 tokens (it would leave most CUs idle:
-    // 512 x 2,048 at 2,048 tokens 51 -> 45 us, at 256 tokens 39 -> 26 us; 2,048 x 4,096 at 256 tokens
-    // 89 -> 48 us)
-    const int t32 = ((a.rows + kGemmBM - 1) / kGemmBM) * ((a.n + 31) / 32);
-    if (q8 && a.n >= kGemmMinN && (a.n <= kSkinnyMaxN || a.rows <= kSkinnyMaxRows || t32 < 256) && a.cols % 32 == 0) {
-        // 16 tokens a workgroup up to 16, 32 up to 32, then 64 (the weights re-read once per token group)
-        const int tt = a.n <= 16 ? 1 : a.n <= 32 ? 2 : 4;
-        const dim3 grid((a.rows + 31) / 32, (a.n + 16 * tt - 1) / (16 * tt));
-        if (tt == 1) hipLaunchKernelGGL((k_mat_skinny<1, 8>), grid, dim3(256), 0, s, a);
-        else if (tt == 2) hipLaunchKernelGGL((k_mat_skinny<2, 4>), grid, dim3(256), 0, s, a);
-        else hipLaunchKernelGGL((k_mat_skinny<4, 2>), grid, dim3(256), 0, s, a);
-        return hipGetLastError();
+    if (q8 && a.n > 1 && tok_wins(a.rows, a.n)) {
+        MatMultiArgs m{};
+        m.m[0] = a, m.count = 1;
+        if (tok_fits(m)) return launch_tok_any(m, s);
     }
     if (a.n >= kGemmMinN && a.cols % 32 == 0) {
         // the widest token tile that still gives two workgroups a CU (fewer weight re-reads), else the
@@ -537,40 +764,40 @@ hipError_t launch_mat(const MatArgs& a, bool q8, hipStream_t s) {
         }
         return hipGetLastError();
     }
-    // matrix-vector: one token a workgroup for a decode step, else four; four rows a wave when that still
-    // gives 256 workgroups a token group, else one (small matrices: more rows in flight at once)
-    const int ntp = a.n == 1 ? 1 : kMatNTP;
+    // matrix-vector: one token a workgroup for a decode step and for Q8 (whose other token counts come here only
+    // with row strides past the token-tile kernel's offsets), else four; four rows a wave when that still gives
+    // 256 workgroups a token group, else one (small matrices: more rows in flight at once)
+    const int ntp = q8 || a.n == 1 ? 1 : kMatNTP;
     const bool rw4 = a.rows >= 4096;
     if ((a.n + ntp - 1) / ntp > 65535) return hipErrorInvalidConfiguration;  // grid y limit (f32, cols % 32 != 0)
     const dim3 grid((a.rows + (rw4 ? 15 : 3)) / (rw4 ? 16 : 4), (a.n + ntp - 1) / ntp), block(256);
     if (q8) {
-        if (ntp == 1) {
-            if (rw4) hipLaunchKernelGGL((k_mat_q8<1, 4>), grid, block, 0, s, a);
-            else hipLaunchKernelGGL((k_mat_q8<1, 1>), grid, block, 0, s, a);
-        } else {
-            if (rw4) hipLaunchKernelGGL((k_mat_q8<kMatNTP, 4>), grid, block, 0, s, a);
-            else hipLaunchKernelGGL((k_mat_q8<kMatNTP, 1>), grid, block, 0, s, a);
-        }
+        if (rw4) hipLaunchKernelGGL((k_mat_q8<4>), grid, block, 0, s, a);
+        else hipLaunchKernelGGL((k_mat_q8<1>), grid, block, 0, s, a);
+    } else if (ntp == 1) {
+        if (rw4) hipLaunchKernelGGL((k_mat_f32<1, 4>), grid, block, 0, s, a);
+        else hipLaunchKernelGGL((k_mat_f32<1, 1>), grid, block, 0, s, a);
     } else {
-        if (ntp == 1) {
-            if (rw4) hipLaunchKernelGGL((k_mat_f32<1, 4>), grid, block, 0, s, a);
-            else hipLaunchKernelGGL((k_mat_f32<1, 1>), grid, block, 0, s, a);
-        } else {
-            if (rw4) hipLaunchKernelGGL((k_mat_f32<kMatNTP, 4>), grid, block, 0, s, a);
-            else hipLaunchKernelGGL((k_mat_f32<kMatNTP, 1>), grid, block, 0, s, a);
-        }
+        if (rw4) hipLaunchKernelGGL((k_mat_f32<kMatNTP, 4>), grid, block, 0, s, a);
+        else hipLaunchKernelGGL((k_mat_f32<kMatNTP, 1>), grid, block, 0, s, a);
     }
     return hipGetLastError();
 }
 
 hipError_t launch_mat_multi(const MatMultiArgs& a0, bool q8, hipStream_t s) {
     const MatArgs& f = a0.m[0];
-    if (f.n >= kGemmMinN && f.cols % 32 == 0) {  // the GEMM: one launch a matrix (each fills the chip)
+    if ((q8 && f.n > 1) || (f.n >= kGemmMinN && f.cols % 32 == 0)) {
+        // the matrices that the token-tile kernel takes in one launch, the GEMM's by themselves (each fills the
+        // chip)
+        MatMultiArgs t{};
         for (int i = 0; i < a0.count; i++) {
-            const hipError_t e = launch_mat(a0.m[i], q8, s);
-            if (e != hipSuccess) return e;
+            if (q8 && tok_wins(a0.m[i].rows, f.n) && tok_fits(a0)) {
+                t.m[t.count++] = a0.m[i];
+            } else if (const hipError_t e = launch_mat(a0.m[i], q8, s); e != hipSuccess) {
+                return e;
+            }
         }
-        return hipSuccess;
+        return t.count ? launch_tok_any(t, s) : hipSuccess;
     }
     MatMultiArgs a = a0;
     int rows = 0;
@@ -586,8 +813,8 @@ hipError_t launch_mat_multi(const MatMultiArgs& a0, bool q8, hipStream_t s) {
     const dim3 grid(wg, (f.n + ntp - 1) / ntp), block(256);
 #define QW_MULTI(Q, N, R) hipLaunchKernelGGL((k_mat_multi<Q, N, R>), grid, block, 0, s, a)
     if (q8) {
-        if (ntp == 1) { if (rw4) QW_MULTI(true, 1, 4); else QW_MULTI(true, 1, 1); }
-        else { if (rw4) QW_MULTI(true, kMatNTP, 4); else QW_MULTI(true, kMatNTP, 1); }
+        if (rw4) QW_MULTI(true, 1, 4);
+        else QW_MULTI(true, 1, 1);
     } else {
         if (ntp == 1) { if (rw4) QW_MULTI(false, 1, 4); else QW_MULTI(false, 1, 1); }
         else { if (rw4) QW_MULTI(false, kMatNTP, 4); else QW_MULTI(false, kMatNTP, 1); }

@@ -286,3 +286,72 @@ def test_mat_multi_f32_equals_separate_calls(qw, oracle, n):
         assert torch.equal(y, ys)
         _check(y.cpu().numpy(), oracle.mat(x, wf=w), np.abs(w), x)
     ctx.close()
+
+
+# The token-tile kernel's shapes: shared rows of four and two blocks (2-4, 5-8 tokens), three parts (9-15), every
+# row-tile and token-tile count its rules pick, four and eight waves, partial row groups, token tiles and quads
+TOK_CASES = [(rows, 160, n) for rows in (45, 2050, 4100, 6200, 9221) for n in (2, 4, 5, 8, 9, 15, 16, 31, 33, 50, 64, 65, 130)]
+TOK_CASES += [(600, 4128, 130), (2050, 4128, 100), (2050, 4128, 200), (90, 32, 3), (90, 32, 70), (33, 1056, 513)]
+
+
+@pytest.mark.parametrize("rows,cols,n", TOK_CASES, ids=lambda v: str(v))
+def test_token_tile_kernel(qw, oracle, rows, cols, n):
+    """Two to 512 tokens on Q8 weights, row strides wider than the rows, nothing stored past rows and tokens.
+
+    Tolerance: below 16 tokens three bf16 parts leave under 2^-26 of |x|, so an output is off by fp32 sums only:
+    4e-6 of sum |W| |x| holds any order of the 160 to 4,128 of them (blocks of 32, then the blocks, then the
+    waves); from 16 tokens two parts leave up to 2^-18."""
+    print(f"token tiles {rows}x{cols} n={n}", flush=True)
+    blocks, _, _ = q8_blocks(101 + rows + n, rows, cols)
+    w8, s = qw.q8_unpack(blocks, rows, cols)
+    x = np.random.default_rng(102 + n).standard_normal((n, cols + 4)).astype(np.float32)
+    ctx = _ctx(qw)
+    y = torch.full((n + 1, rows + 5), 7.0, device=DEV)
+    ctx.mat(dev(x)[:, :cols], y[:n, :rows], dev(w8), dev(s))
+    torch.cuda.synchronize()
+    got = y.cpu().numpy()
+    x = x[:, :cols]
+    mag = np.abs(w8.astype(np.float32) * np.repeat(s, 32, axis=1)).astype(np.float64) @ np.abs(x.astype(np.float64)).T
+    err = np.abs(got[:n, :rows].astype(np.float64) - oracle.mat(x, w8=w8, s=s))
+    assert np.all(err <= (4e-6 if n < 16 else 1e-5) * mag.T + 1e-6), float((err / mag.T).max())
+    assert np.all(got[n] == 7.0) and np.all(got[:, rows:] == 7.0)
+    ctx.close()
+
+
+@pytest.mark.parametrize("n", [3, 7, 12])
+def test_token_tile_infinities(qw, n):
+    """Infinite and NaN inputs below 16 tokens reach the outputs as fp32 products would have them, and only their
+    own token's."""
+    rows, cols = 40, 96
+    blocks, _, _ = q8_blocks(110, rows, cols)
+    w8, s = qw.q8_unpack(blocks, rows, cols)
+    x = np.random.default_rng(111).standard_normal((n, cols)).astype(np.float32)
+    x[0, 5], x[1, 70], x[n - 1, 33] = np.inf, -np.inf, np.nan
+    ctx = _ctx(qw)
+    y = torch.zeros((n, rows), device=DEV)
+    ctx.mat(dev(x), y, dev(w8), dev(s))
+    torch.cuda.synchronize()
+    with np.errstate(invalid="ignore"):
+        want = x.astype(np.float64) @ (w8 * np.repeat(s.astype(np.float64), 32, axis=1)).T
+    np.testing.assert_allclose(y.cpu().numpy(), want, rtol=1e-4, atol=1e-4)
+    ctx.close()
+
+
+@pytest.mark.parametrize("n", [3, 20])
+def test_mat_wide_row_stride(qw, oracle, n):
+    """Token rows too far apart for the token-tile kernel's offsets go to the other kernels."""
+    rows, cols, stride = 70, 64, 6_400_004
+    blocks, _, _ = q8_blocks(112, rows, cols)
+    w8, s = qw.q8_unpack(blocks, rows, cols)
+    x = np.random.default_rng(113).standard_normal((n, cols)).astype(np.float32)
+    xd = torch.zeros(stride * n, device=DEV).view(n, stride)[:, :cols]
+    xd.copy_(dev(x))
+    ctx = _ctx(qw)
+    wd, sd = dev(w8), dev(s)
+    y, y2 = torch.zeros((n, rows), device=DEV), torch.zeros((n, rows), device=DEV)
+    ctx.mat(xd, y, wd, sd)
+    ctx.mat_multi(xd, [(y2, wd, sd)])
+    torch.cuda.synchronize()
+    _check(y.cpu().numpy(), oracle.mat(x, w8=w8, s=s), np.abs(w8.astype(np.float32) * np.repeat(s, 32, axis=1)), x)
+    assert torch.equal(y, y2)
+    ctx.close()
