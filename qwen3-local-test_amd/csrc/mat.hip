@@ -16,6 +16,7 @@
 // issued before the first is used. A 16-column group never crosses a 32-weight block, so the lane applies its
 // block scale once per group. The partial dot products are summed over the wave with DPP row operations and
 // permlane swaps.
+#include <algorithm>
 #include <atomic>
 
 #include "common.hpp"
@@ -182,18 +183,15 @@ __global__ __launch_bounds__(256) void k_mat_multi(MatMultiArgs a) {
     else mat_f32_body<NTP, RW>(a.m[i], bx);
 }
 
-// ---- many tokens: tiled MFMA GEMM ------------------------------------------------------------------
-// Replaces the q4_gemm_q8 / q4_gemm_f32 pipelines (shaders/q4_gemm.comp) that Qwen4Vulkan::mat selects from
-// nine tokens on (src/qwen4_vk.cpp:852-853). A workgroup owns a 128-row x BN-token tile of Y, walks the
-// columns one 32-column step at a time (one Q8 block) through two LDS stages, and its four waves each own a
-// 64-row x BN/2-token quarter as 4 x BN/32 v_mfma_f32_16x16x32_bf16 tiles (A = weight rows, B = token rows).
-// fp32 accuracy from bf16 products: an int8 weight is exact in bf16, and an fp32 x is split into
-// x_hi = bf16(x) and x_lo = bf16(x - x_hi), which leaves |x - x_hi - x_lo| <= 2^-18 |x|; a product's two
-// MFMAs then carry it to within 2^-18 |w x| before the fp32 accumulation. Q8: each 32-column step's
-// product (a fresh accumulator) is scaled by its rows' block scales into the running sum, as the reference
-// applies the scale per block. f32 weights are split the same way (four MFMAs a tile: hi.hi, hi.lo,
-// lo.hi, lo.lo). The next step's global loads are in flight while the current step's MFMAs run; tiles are
-// assigned so that each XCD takes a contiguous range of row tiles (its weights stay in its L2).
+// ---- fp32 weights, many tokens: tiled MFMA GEMM ---------------------------------------------------------
+// Replaces the q4_gemm_f32 pipeline (shaders/q4_gemm.comp) that Qwen4Vulkan::mat selects from nine tokens on
+// (src/qwen4_vk.cpp:852-853). A workgroup owns a 128-row x BN-token tile of Y, walks the columns one 32-column
+// step at a time through two LDS stages, and its four waves each own a 64-row x BN/2-token quarter as
+// 4 x BN/32 v_mfma_f32_16x16x32_bf16 tiles (A = weight rows, B = token rows). fp32 accuracy from bf16 products:
+// an fp32 value v is split into hi = bf16(v) and lo = bf16(v - hi), which leaves |v - hi - lo| <= 2^-18 |v|; four
+// MFMAs a tile (hi.hi, hi.lo, lo.hi, lo.lo) then carry a product to within 2^-17 before the fp32 accumulation.
+// The next step's global loads are in flight while the current step's MFMAs run; tiles are assigned so that each
+// XCD takes a contiguous range of row tiles (its weights stay in its L2).
 constexpr int kGemmBM = 128;  // rows a workgroup
 
 // Byte offset of 16-byte chunk g (k = 8 g .. 8 g + 7) of tile row r in an LDS tile of [rows][32] bf16: the
@@ -230,6 +228,17 @@ __device__ __forceinline__ void split_bf16(const float (&v)[8], bf16x8& hi, bf16
 // token counts below 16.
 __device__ __forceinline__ uint32_t pk_bf16(float a, float b) {  // one v_cvt_pk_bf16_f32
     return __builtin_bit_cast(uint32_t, __builtin_convertvector(f32x2{a, b}, bf16x2));
+}
+
+// What the bf16 pair w = pk_bf16(v0, v1) leaves of v0 (E = 0) or v1 (E = 1), exactly, in one v_dot2_f32_bf16 with
+// (-1, 0) or (0, -1) (an infinity in either makes both NaN). The pair is made opaque: as a constant the compiler
+// writes the first as the inline operand -1.0, which the instruction reads as the second.
+template <int E>
+__device__ __forceinline__ float rest_bf16(uint32_t w, float v) {
+    uint32_t m;
+    if constexpr (E == 0) asm("s_mov_b32 %0, 0xbf80" : "=s"(m));
+    else asm("s_mov_b32 %0, 0xbf800000" : "=s"(m));
+    return __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(bf16x2, w), __builtin_bit_cast(bf16x2, m), v, false);
 }
 
 // Eight int8 weights (two words) as bf16, exactly.
@@ -363,11 +372,13 @@ __device__ __forceinline__ void mat_tok_body(const MatArgs& a, int bx, int by, u
                         for (int k = 0; k < NS; k++) {
                             const uint32_t w = pk_bf16(v0, v1);
                             part[k][e] = w;
-                            if (k + 1 < NS) {
-                                const float h0 = __uint_as_float(w << 16), h1 = __uint_as_float(w & 0xFFFF0000u);
+                            if (NS == 3 && k == 0) {
                                 // three parts: an infinity is its first part (as fp32 products would have it)
-                                v0 = NS == 3 && k == 0 && __builtin_fabsf(h0) == __builtin_inff() ? 0.f : v0 - h0;
-                                v1 = NS == 3 && k == 0 && __builtin_fabsf(h1) == __builtin_inff() ? 0.f : v1 - h1;
+                                const float h0 = __uint_as_float(w << 16), h1 = __uint_as_float(w & 0xFFFF0000u);
+                                v0 = __builtin_fabsf(h0) == __builtin_inff() ? 0.f : v0 - h0;
+                                v1 = __builtin_fabsf(h1) == __builtin_inff() ? 0.f : v1 - h1;
+                            } else if (k + 1 < NS) {
+                                v0 = rest_bf16<0>(w, v0), v1 = rest_bf16<1>(w, v1);
                             }
                         }
                     }
@@ -471,12 +482,12 @@ __global__ __launch_bounds__(64 * KW) void k_mat_tok(MatMultiArgs a) {
     mat_tok_body<TT, R, NS, B, KW>(a.m[i], (int)blockIdx.x - (i ? a.wg_end[i - 1] : 0), blockIdx.y, smem);
 }
 
-template <bool Q8, int BN>
+template <int BN>
 __global__ __launch_bounds__(256, 2) void k_gemm(MatArgs a) {
     constexpr int NT = BN / 32;                      // 16-token tiles a wave (BN = 32, 64 or 128)
     constexpr int W_B = kGemmBM * 64;                // one bf16 weight plane of a stage
     constexpr int X_B = BN * 64;                     // one bf16 token plane
-    constexpr int STAGE = (Q8 ? W_B + kGemmBM * 4 : 2 * W_B) + 2 * X_B;
+    constexpr int STAGE = 2 * W_B + 2 * X_B;
     __shared__ __attribute__((aligned(16))) unsigned char smem[2 * STAGE];
     const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, c = lane & 15, g = lane >> 4;
     const int wr = wave & 1, wt = wave >> 1;
@@ -498,23 +509,16 @@ __global__ __launch_bounds__(256, 2) void k_gemm(MatArgs a) {
 
     // one step's global data in registers
     struct Pre {
-        u32x4 w;       // Q8: 16 int8 weights
-        float f[16];   // f32: 16 weights
-        float sc;      // Q8: block scale of row `tid` (threads 0..127)
+        float f[16];   // weights
         float x[XC];
     };
     auto load = [&](Pre& P, int kb) {
         const int k0 = kb * 32;
-        if constexpr (Q8) {
-            P.w = *reinterpret_cast<const u32x4*>(static_cast<const int8_t*>(a.w) + wrow * a.cols + k0 + 16 * lh);
-            if (tid < kGemmBM) P.sc = a.s[(size_t)min(r0 + tid, a.rows - 1) * nkb + kb];
-        } else {
-            const float* wp = static_cast<const float*>(a.w) + wrow * a.cols + k0 + 16 * lh;
+        const float* wp = static_cast<const float*>(a.w) + wrow * a.cols + k0 + 16 * lh;
 #pragma unroll
-            for (int i = 0; i < 16; i += 4) {
-                const f32x4 v = *reinterpret_cast<const f32x4*>(wp + i);
-                P.f[i] = v[0], P.f[i + 1] = v[1], P.f[i + 2] = v[2], P.f[i + 3] = v[3];
-            }
+        for (int i = 0; i < 16; i += 4) {
+            const f32x4 v = *reinterpret_cast<const f32x4*>(wp + i);
+            P.f[i] = v[0], P.f[i + 1] = v[1], P.f[i + 2] = v[2], P.f[i + 3] = v[3];
         }
         if (xl) {
 #pragma unroll
@@ -526,29 +530,15 @@ __global__ __launch_bounds__(256, 2) void k_gemm(MatArgs a) {
     };
     auto store = [&](const Pre& P, int st) {
         unsigned char* S = smem + st * STAGE;
-        if constexpr (Q8) {
 #pragma unroll
-            for (int h = 0; h < 2; h++) {
-                bf16x8 v;
+        for (int h = 0; h < 2; h++) {
+            float v8[8];
 #pragma unroll
-                for (int j = 0; j < 8; j++) {
-                    const int q = (int)P.w[2 * h + j / 4];
-                    v[j] = (__bf16)(float)((q << (24 - 8 * (j % 4))) >> 24);
-                }
-                *reinterpret_cast<bf16x8*>(S + gemm_off(lr, 2 * lh + h)) = v;
-            }
-            if (tid < kGemmBM) reinterpret_cast<float*>(S + W_B + 2 * X_B)[tid] = P.sc;
-        } else {
-#pragma unroll
-            for (int h = 0; h < 2; h++) {
-                float v8[8];
-#pragma unroll
-                for (int j = 0; j < 8; j++) v8[j] = P.f[8 * h + j];
-                bf16x8 hi, lo;
-                split_bf16(v8, hi, lo);
-                *reinterpret_cast<bf16x8*>(S + gemm_off(lr, 2 * lh + h)) = hi;
-                *reinterpret_cast<bf16x8*>(S + W_B + 2 * X_B + gemm_off(lr, 2 * lh + h)) = lo;
-            }
+            for (int j = 0; j < 8; j++) v8[j] = P.f[8 * h + j];
+            bf16x8 hi, lo;
+            split_bf16(v8, hi, lo);
+            *reinterpret_cast<bf16x8*>(S + gemm_off(lr, 2 * lh + h)) = hi;
+            *reinterpret_cast<bf16x8*>(S + W_B + 2 * X_B + gemm_off(lr, 2 * lh + h)) = lo;
         }
 #pragma unroll
         for (int h = 0; h < XC / 8; h++) {
@@ -581,30 +571,15 @@ __global__ __launch_bounds__(256, 2) void k_gemm(MatArgs a) {
             Bh[t] = *reinterpret_cast<const bf16x8*>(S + W_B + gemm_off(r, g));
             Bl[t] = *reinterpret_cast<const bf16x8*>(S + W_B + X_B + gemm_off(r, g));
         }
-        if constexpr (Q8) {
-            const float* sS = reinterpret_cast<const float*>(S + W_B + 2 * X_B);
 #pragma unroll
-            for (int m = 0; m < 4; m++) {
-                const f32x4 sc = *reinterpret_cast<const f32x4*>(sS + wr * 64 + m * 16 + 4 * g);
+        for (int m = 0; m < 4; m++) {
+            const bf16x8 Al = *reinterpret_cast<const bf16x8*>(S + W_B + 2 * X_B + gemm_off(wr * 64 + m * 16 + c, g));
 #pragma unroll
-                for (int t = 0; t < NT; t++) {
-                    f32x4 p = __builtin_amdgcn_mfma_f32_16x16x32_bf16(A[m], Bh[t], f32x4{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
-                    p = __builtin_amdgcn_mfma_f32_16x16x32_bf16(A[m], Bl[t], p, 0, 0, 0);
-#pragma unroll
-                    for (int i = 0; i < 4; i++) acc[m][t][i] = __builtin_fmaf(sc[i], p[i], acc[m][t][i]);
-                }
-            }
-        } else {
-#pragma unroll
-            for (int m = 0; m < 4; m++) {
-                const bf16x8 Al = *reinterpret_cast<const bf16x8*>(S + W_B + 2 * X_B + gemm_off(wr * 64 + m * 16 + c, g));
-#pragma unroll
-                for (int t = 0; t < NT; t++) {
-                    acc[m][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(A[m], Bh[t], acc[m][t], 0, 0, 0);
-                    acc[m][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(A[m], Bl[t], acc[m][t], 0, 0, 0);
-                    acc[m][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(Al, Bh[t], acc[m][t], 0, 0, 0);
-                    acc[m][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(Al, Bl[t], acc[m][t], 0, 0, 0);
-                }
+            for (int t = 0; t < NT; t++) {
+                acc[m][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(A[m], Bh[t], acc[m][t], 0, 0, 0);
+                acc[m][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(A[m], Bl[t], acc[m][t], 0, 0, 0);
+                acc[m][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(Al, Bh[t], acc[m][t], 0, 0, 0);
+                acc[m][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(Al, Bl[t], acc[m][t], 0, 0, 0);
             }
         }
     };
@@ -644,25 +619,237 @@ __global__ __launch_bounds__(256, 2) void k_gemm(MatArgs a) {
     }
 }
 
+// ---- Q8, many tokens: tiled MFMA GEMM ---------------------------------------------------------------
+// Replaces the q4_gemm_q8 pipeline (shaders/q4_gemm.comp) that Qwen4Vulkan::mat selects from nine tokens on
+// (src/qwen4_vk.cpp:852-853).
+// A workgroup of eight waves owns a tile of BM = 32 RT GR rows x BN = 32 TT GT tokens, each wave 32 RT x 32 TT of
+// it, and walks the columns 64 (two Q8 blocks) at a time through two LDS stages: per 32-column block and 32 x 32
+// piece four v_mfma_f32_32x32x16_bf16 (two column halves of the hi, then of the lo part of x; the weights exact
+// in bf16, the B operand) into a fresh accumulator that is scaled by the lane's row's block scale into the
+// running sum.
+//
+// What bounds it is a SIMD's issue: per MFMA eight other vector instructions (half of them the scaling, the rest
+// the conversion of int8 and fp32 to bf16), and the two share it: 32x32x16 with eight of them 18.7 ns (14.2 with
+// none), 16x16x32, half the work, with four 14.4 ns (8.3 with none). Then the step's barrier and operand reads,
+// which both waves of a SIMD wait for together. 8,192 x 2,048 at 2,048 tokens, one box: 200 us with 128 x 128
+// tiles of four waves a workgroup and token rows loaded two lanes a row; 148 with rows loaded by consecutive
+// lanes and 256 x 128 tiles, alike with 16x16x32 MFMAs in the compiler's order or pinned; 147 with 32x32x16, of
+// which the conversions take 30 and the scaling, by leaving three quarters of it out, 18.
+template <int RT, int TT, int GR, int GT>
+__global__ __launch_bounds__(512) void k_gemm_q8(MatArgs a) {
+    static_assert(GR * GT == 8, "eight waves");
+    constexpr int BM = 32 * RT * GR, BN = 32 * TT * GT;
+    constexpr int WL = BM / 128, XL = BN / 32;  // 16-byte loads a thread and step: weights, token rows
+    constexpr int W_B = BM * 128, X_B = BN * 128, STAGE = W_B + 2 * X_B + BM * 8;
+    extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
+    const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
+    const int c = lane & 31, h = lane >> 5;
+    const int wr = (wave % GR) * 32 * RT, wt = (wave / GR) * 32 * TT;
+
+    const int RTs = (a.rows + BM - 1) / BM, TTs = (a.n + BN - 1) / BN, T = RTs * TTs;
+    const int b = blockIdx.x;
+    const int idx = (T & 7) ? b : (b & 7) * (T >> 3) + (b >> 3);  // XCD b % 8 takes tiles [x T/8, (x+1) T/8)
+    const int r0 = (idx / TTs) * BM, t0 = (idx % TTs) * BN;
+    const int nkb = a.cols >> 5, nst = (nkb + 1) >> 1;
+
+    // loads by consecutive lanes: four lanes a weight row's 64 columns, sixteen a token's, the step and the load's
+    // first row in the scalar offset. Rows and tokens past the ends, and a last half step's second block (kFar
+    // added), lie outside the resources and read zero.
+    constexpr unsigned kFar = 0x60000000u;
+    const int wq = tid & 3, xq = tid & 15;
+    const int nr = min(BM, a.rows - r0), nt = min(BN, a.n - t0);
+    const __amdgpu_buffer_rsrc_t rw = __builtin_amdgcn_make_buffer_rsrc(
+        const_cast<int8_t*>(static_cast<const int8_t*>(a.w)) + (size_t)r0 * a.cols, (short)0, nr * a.cols, 0x00020000);
+    const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc(
+        const_cast<float*>(a.s) + (size_t)r0 * nkb, (short)0, nr * nkb * 4, 0x00020000);
+    const __amdgpu_buffer_rsrc_t rx = __builtin_amdgcn_make_buffer_rsrc(
+        const_cast<float*>(a.x) + (size_t)t0 * a.x_stride, (short)0, ((nt - 1) * a.x_stride + a.cols) * 4, 0x00020000);
+    const unsigned wo = (tid >> 2) * a.cols + 16 * wq, xo = ((tid >> 4) * a.x_stride + 4 * xq) * 4;
+    const unsigned so = ((tid >> 1) % BM * nkb + (tid & 1)) * 4;
+    u32x4 wv[WL];
+    f32x4 xv[XL];
+    float sv;
+    auto load_w = [&](int k) {
+        const unsigned o = 2 * k + (wq >> 1) < nkb ? wo : wo + kFar;
+#pragma unroll
+        for (int i = 0; i < WL; i++)
+            wv[i] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(rw, (int)o, 128 * i * a.cols + 64 * k, 0));
+        sv = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(rs, (int)so, 8 * k, 0));
+    };
+    auto load_x = [&](int k, int i) {
+        const unsigned o = 2 * k + (xq >> 3) < nkb ? xo : xo + kFar;
+        xv[i] = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(rx, (int)o, 128 * i * a.x_stride + 256 * k, 0));
+    };
+    // LDS rows of 64 columns are eight 16-byte chunks, chunk q of row r at q ^ (r / 2) % 8: operand reads (16
+    // rows' chunk q) and the loaders' writes are free of bank conflicts
+    auto at = [](int r, int q) { return r * 128 + ((q ^ ((r >> 1) & 7)) << 4); };
+    // the conversion of the loaded pieces in units of a few instructions: four to each half of a weight piece (its
+    // pairs of weights), two to a token piece
+    constexpr int UW = 8 * WL, U = UW + 2 * XL;
+    uint32_t cw[4], ch[2], cl[2];
+    auto unit = [&](int u, unsigned char* S) {
+        if (u < UW) {
+            const int i = u / 8, hf = u / 4 % 2, e = u % 4;
+            const int v = (int)wv[i][2 * hf + e / 2], sh = 16 * (e & 1);
+            cw[e] = pk_bf16((float)((v << (24 - sh)) >> 24), (float)((v << (16 - sh)) >> 24));
+            if (e == 3) *reinterpret_cast<u32x4*>(S + at(128 * i + (tid >> 2), 2 * wq + hf)) = u32x4{cw[0], cw[1], cw[2], cw[3]};
+        } else {
+            const int i = (u - UW) / 2, e = (u - UW) % 2;
+            const float v0 = xv[i][2 * e], v1 = xv[i][2 * e + 1];
+            ch[e] = pk_bf16(v0, v1);
+            cl[e] = pk_bf16(rest_bf16<0>(ch[e], v0), rest_bf16<1>(ch[e], v1));
+            if (e == 1) {
+                unsigned char* d = S + W_B + at(32 * i + (tid >> 4), xq >> 1) + 8 * (xq & 1);
+                *reinterpret_cast<u32x2*>(d) = u32x2{ch[0], ch[1]};
+                *reinterpret_cast<u32x2*>(d + X_B) = u32x2{cl[0], cl[1]};
+            }
+        }
+    };
+    // the scale of a block past the row is 0: a last half step's second block adds nothing
+    auto put_s = [&](int k, unsigned char* S) {
+        if (tid < 2 * BM)
+            reinterpret_cast<float*>(S + W_B + 2 * X_B)[(tid & 1) * BM + (tid >> 1)] = 2 * k + (tid & 1) < nkb ? sv : 0.f;
+    };
+
+    f32x16 acc[RT][TT];
+#pragma unroll
+    for (int r = 0; r < RT; r++)
+#pragma unroll
+        for (int t = 0; t < TT; t++)
+#pragma unroll
+            for (int e = 0; e < 16; e++) acc[r][t][e] = 0.f;
+
+    load_w(0);
+#pragma unroll
+    for (int i = 0; i < XL; i++) load_x(0, i);
+#pragma unroll
+    for (int u = 0; u < U; u++) unit(u, smem);
+    put_s(0, smem);
+    load_w(min(1, nst - 1));
+#pragma unroll
+    for (int i = 0; i < XL; i++) load_x(min(1, nst - 1), i);
+    __syncthreads();
+    // Stage k % 2 holds step k; while its MFMAs run, step k + 1 (loaded a step ago) is converted into the other
+    // stage, whose last readers passed the previous barrier, and step k + 2's loads follow each piece. A step is
+    // 2 TT RT passes (block j, token tile t, row tile r) of four slots: one MFMA, the scaling of a quarter of the
+    // pass before, a conversion unit or so, pinned in this order so that a wave's MFMAs and its other
+    // instructions take turns. The step past the last is converted too, unread.
+    constexpr int P = 2 * TT * RT, SL = 4 * P;
+    bf16x8 W[2][RT][2], xf[2][2][2];  // [block][row tile][column half]; [(j, t) parity][part][column half]
+    float sc[2][RT];
+    f32x16 d[2];
+#pragma unroll
+    for (int e = 0; e < 16; e++) d[1][e] = 0.f;
+#pragma unroll
+    for (int r = 0; r < RT; r++) sc[1][r] = 0.f;
+#pragma unroll 1
+    for (int k = 0; k < nst; k++) {
+        const unsigned char* S = smem + (k & 1) * STAGE;
+        unsigned char* N = smem + ((k + 1) & 1) * STAGE;
+        const float* sS = reinterpret_cast<const float*>(S + W_B + 2 * X_B);
+        const int k2 = min(k + 2, nst - 1);
+        auto read_w = [&](int j, int r, int q) {
+            W[j][r][q] = *reinterpret_cast<const bf16x8*>(S + at(wr + 32 * r + c, 4 * j + 2 * q + h));
+        };
+        auto read_x = [&](int jt, int part, int q) {
+            xf[jt & 1][part][q] = *reinterpret_cast<const bf16x8*>(
+                S + W_B + part * X_B + at(wt + 32 * (jt % TT) + c, 4 * (jt / TT) + 2 * q + h));
+        };
+#pragma unroll
+        for (int q = 0; q < 2; q++) read_w(0, 0, q), read_x(0, 0, q);
+#pragma unroll
+        for (int q = 0; q < 2; q++) read_x(0, 1, q);
+#pragma unroll
+        for (int r = 1; r < RT; r++) read_w(0, r, 0), read_w(0, r, 1);
+        static_for<0, SL>([&](auto s_) {
+            constexpr int s = s_, p = s / 4, q4 = s % 4;
+            constexpr int r = p % RT, jt = p / RT, t = jt % TT, j = jt / TT;
+            constexpr int pp = (p + P - 1) % P, pr = pp % RT, pt = pp / RT % TT, pj = pp / RT / TT;  // the pass before
+            constexpr int part = q4 / 2, q = q4 % 2;
+            const f32x16 zero = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+            d[p & 1] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(xf[jt & 1][part][q], W[j][r][q], q4 ? d[p & 1] : zero, 0, 0, 0);
+            // (none in the first slot: the pass before's last MFMA has not ended yet)
+            constexpr int f0 = q4 < 2 ? 0 : 5 * q4 - 4, f1 = q4 == 0 ? 0 : 5 * q4 + 1;
+#pragma unroll
+            for (int e = f0; e < f1; e++) {
+                float v = __builtin_fmaf(sc[pj][pr], d[(p + 1) & 1][e], acc[pr][pt][e]);
+                asm volatile("" : "+v"(v));  // here, not sunk to the step's end
+                acc[pr][pt][e] = v;
+            }
+            // units: the pass's first two thirds in its first slot, the rest in its last
+            constexpr int u0 = p * U / P, u2 = (p + 1) * U / P, u1 = u0 + (2 * (u2 - u0) + 2) / 3;
+            static_for<q4 == 0 ? u0 : u1, q4 == 0 ? u1 : q4 == 3 ? u2 : u1>([&](auto u_) {
+                constexpr int u = u_;
+                unit(u, N);
+                if constexpr (u == UW - 1) {
+                    put_s(k + 1, N);
+                    load_w(k2);
+                }
+                if constexpr (u >= UW && (u - UW) % 2 == 1) load_x(k2, (u - UW) / 2);
+            });
+            // the next token tile's operands and the second block's weights ahead of their passes; the scales of
+            // this step's blocks once the last pass of the step before has used its own
+            if constexpr (r == RT - 1 && jt + 1 < 2 * TT) read_x(jt + 1, q4 / 2, q4 % 2);
+            if constexpr (j == 0 && t == TT - 1 && q4 < 2) read_w(1, r, q4);
+            if constexpr (p == 0 && q4 == 3) {
+#pragma unroll
+                for (int i = 0; i < RT; i++) sc[0][i] = sS[wr + 32 * i + c], sc[1][i] = sS[BM + wr + 32 * i + c];
+            }
+            __builtin_amdgcn_sched_barrier(0);
+        });
+        __syncthreads();
+    }
+#pragma unroll
+    for (int e = 0; e < 16; e++)
+        acc[RT - 1][TT - 1][e] = __builtin_fmaf(sc[1][RT - 1], d[1][e], acc[RT - 1][TT - 1][e]);
+
+    // lane (c, h): row 32 r + c of the wave's, tokens 32 t + 8 (e / 4) + 4 h + e % 4
+#pragma unroll
+    for (int t = 0; t < TT; t++)
+#pragma unroll
+        for (int e = 0; e < 16; e++) {
+            const int tok = t0 + wt + 32 * t + 8 * (e / 4) + 4 * h + e % 4;
+            if (tok >= a.n) continue;
+            float* yr = a.y + (size_t)tok * a.y_stride;
+#pragma unroll
+            for (int r = 0; r < RT; r++) {
+                const int row = r0 + wr + 32 * r + c;
+                float v = acc[r][t][e];
+                if (a.post == 1) {
+                    const float u = v * a.post_scale;
+                    v = u / (1.0f + __expf(-u));
+                }
+                if (row < a.rows) yr[row] = v;
+            }
+        }
+}
+
+template <int RT, int TT, int GR, int GT>
+constexpr size_t gemm_lds() {
+    return 2 * (32 * RT * GR * 136 + 2 * 32 * TT * GT * 128);
+}
+
 }  // namespace
 
 namespace {
 
+// Raises a kernel's dynamic LDS past the default 64 KB, once per device (`raised`: a bit each).
+hipError_t raise_lds(const void* kernel, size_t lds, std::atomic<uint64_t>& raised) {
+    if (lds <= 64 * 1024) return hipSuccess;
+    int dev = 0;
+    if (hipGetDevice(&dev) != hipSuccess) return hipErrorInvalidDevice;
+    const uint64_t bit = 1ull << (dev & 63);
+    if (raised.load(std::memory_order_acquire) & bit) return hipSuccess;
+    const hipError_t e = hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+    if (e == hipSuccess) raised.fetch_or(bit, std::memory_order_acq_rel);
+    return e;
+}
+
 template <int TT, int R, int NS, int B, int KW>
 hipError_t launch_tok(MatMultiArgs a, hipStream_t s) {
     constexpr size_t lds = tok_lds<TT, R, NS, B, KW>();
-    if constexpr (lds > 64 * 1024) {  // past the default limit: raised once per device
-        static std::atomic<uint64_t> raised{0};
-        int dev = 0;
-        if (hipGetDevice(&dev) != hipSuccess) return hipErrorInvalidDevice;
-        const uint64_t bit = 1ull << (dev & 63);
-        if (!(raised.load(std::memory_order_acquire) & bit)) {
-            const hipError_t e = hipFuncSetAttribute((const void*)k_mat_tok<TT, R, NS, B, KW>,
-                                                     hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-            if (e != hipSuccess) return e;
-            raised.fetch_or(bit, std::memory_order_acq_rel);
-        }
-    }
+    static std::atomic<uint64_t> raised{0};
+    if (const hipError_t e = raise_lds((const void*)k_mat_tok<TT, R, NS, B, KW>, lds, raised); e != hipSuccess) return e;
     int wg = 0;
     for (int i = 0; i < a.count; i++) a.wg_end[i] = wg += (a.m[i].rows + 16 * R - 1) / (16 * R);
     hipLaunchKernelGGL((k_mat_tok<TT, R, NS, B, KW>), dim3(wg, (a.m[0].n + 16 * TT - 1) / (16 * TT)), dim3(64 * KW), lds, s, a);
@@ -687,12 +874,6 @@ constexpr TokShape kTok8[] = {{1, 1, launch_tok<1, 1, 2, 1, 8>}, {1, 2, launch_t
 constexpr TokShape kTok4[] = {{1, 2, launch_tok<1, 2, 2, 1, 4>}, {1, 4, launch_tok<1, 4, 2, 1, 4>},
                               {2, 4, launch_tok<2, 4, 2, 1, 4>}};
 constexpr int kCus = 256;
-
-// Whether a Q8 matrix takes the token-tile kernel (from two tokens): up to 512 tokens, at any count for matrices
-// of up to 1,024 rows, and wherever the GEMM would have fewer than 256 tiles of 128 rows x 32 tokens.
-bool tok_wins(int rows, int n) {
-    return n <= 512 || rows <= 1024 || ((rows + kGemmBM - 1) / kGemmBM) * ((n + 31) / 32) < 256;
-}
 
 // Row groups of 16 R rows, every matrix by itself.
 int row_groups(const MatMultiArgs& a, int r) {
@@ -737,31 +918,69 @@ hipError_t launch_tok_any(const MatMultiArgs& a, hipStream_t s) {
     return k->launch(a, s);
 }
 
+template <int RT, int TT, int GR, int GT>
+hipError_t launch_gemm_q8(const MatArgs& a, hipStream_t s) {
+    constexpr size_t lds = gemm_lds<RT, TT, GR, GT>();
+    static std::atomic<uint64_t> raised{0};
+    if (const hipError_t e = raise_lds((const void*)k_gemm_q8<RT, TT, GR, GT>, lds, raised); e != hipSuccess) return e;
+    const int bm = 32 * RT * GR, bn = 32 * TT * GT;
+    hipLaunchKernelGGL((k_gemm_q8<RT, TT, GR, GT>), dim3(((a.rows + bm - 1) / bm) * ((a.n + bn - 1) / bn)), dim3(512), lds, s, a);
+    return hipGetLastError();
+}
+
+// The Q8 GEMM's tiles with what a 64-column step of one takes a CU, in hundredths of a microsecond (one tile a CU;
+// 2,048 tokens through 8,192 x 2,048 and 2,048 x 4,096: 147 / 183 / 216 and 109 / 85 / 103 us).
+struct GemmTile {
+    int bm, bn, step;
+    hipError_t (*launch)(const MatArgs&, hipStream_t);
+};
+constexpr GemmTile kGemmTiles[] = {{256, 128, 235, launch_gemm_q8<2, 2, 4, 2>},
+                                   {128, 128, 135, launch_gemm_q8<2, 1, 2, 4>},
+                                   {128, 64, 82, launch_gemm_q8<1, 1, 4, 2>}};
+int gemm_cost(const GemmTile& t, int rows, int n) {
+    const long long tiles = (long long)((rows + t.bm - 1) / t.bm) * ((n + t.bn - 1) / t.bn);
+    return (int)std::min<long long>((tiles + kCus - 1) / kCus * t.step, 1 << 30);
+}
+const GemmTile& gemm_tile(int rows, int n) {
+    const GemmTile* best = kGemmTiles;
+    for (const GemmTile& t : kGemmTiles)
+        if (gemm_cost(t, rows, n) < gemm_cost(*best, rows, n)) best = &t;
+    return *best;
+}
+// Whether the Q8 GEMM's 32-bit offsets reach the operands.
+bool gemm_fits(const MatArgs& a) { return a.cols <= 1 << 22 && (127ll * a.x_stride + a.cols) * 4 < 0x60000000ll; }
+
+// Whether a Q8 matrix takes the token-tile kernel (from two tokens on): up to 64 tokens, else where its 64-row x
+// 32-token workgroups, two a CU and 0.55 us a pair and 64 columns, take less than the GEMM's tiles (8,192 x 2,048
+// at 128 / 256 / 512 tokens 29 / 37 / 68 us against 29 / 31 / 48; 2,048 x 4,096 at 256 / 512 / 777 20 / 36 / 64
+// against 50 / 51 / 53; 512 x 2,048 at 2,048 26 against 28). By the matrix alone, so that qwattn_mat and
+// qwattn_mat_multi agree.
+bool tok_wins(const MatArgs& a) {
+    if (a.n <= 64) return true;
+    const long long wgs = (long long)((a.rows + 63) / 64) * ((a.n + 31) / 32);
+    return std::max<long long>(55, 55 * wgs / (2 * kCus)) <= gemm_cost(gemm_tile(a.rows, a.n), a.rows, a.n);
+}
+
 }  // namespace
 
 hipError_t launch_mat(const MatArgs& a, bool q8, hipStream_t s) {
-    if (q8 && a.n > 1 && tok_wins(a.rows, a.n)) {
+    if (q8 && a.n > 1) {
         MatMultiArgs m{};
         m.m[0] = a, m.count = 1;
-        if (tok_fits(m)) return launch_tok_any(m, s);
+        const bool gemm = gemm_fits(a);
+        if (tok_fits(m) && (!gemm || tok_wins(a))) return launch_tok_any(m, s);
+        if (gemm) return gemm_tile(a.rows, a.n).launch(a, s);
     }
-    if (a.n >= kGemmMinN && a.cols % 32 == 0) {
+    if (!q8 && a.n >= kGemmMinN && a.cols % 32 == 0) {
         // the widest token tile that still gives two workgroups a CU (fewer weight re-reads), else the
         // narrowest (the most workgroups)
         const int rt = (a.rows + kGemmBM - 1) / kGemmBM;
         const auto tiles = [&](int bn) { return rt * ((a.n + bn - 1) / bn); };
         const int bn = tiles(128) >= 512 ? 128 : tiles(64) >= 512 ? 64 : 32;
         const dim3 grid(tiles(bn)), block(256);
-        if (bn == 128) {
-            if (q8) hipLaunchKernelGGL((k_gemm<true, 128>), grid, block, 0, s, a);
-            else hipLaunchKernelGGL((k_gemm<false, 128>), grid, block, 0, s, a);
-        } else if (bn == 64) {
-            if (q8) hipLaunchKernelGGL((k_gemm<true, 64>), grid, block, 0, s, a);
-            else hipLaunchKernelGGL((k_gemm<false, 64>), grid, block, 0, s, a);
-        } else {
-            if (q8) hipLaunchKernelGGL((k_gemm<true, 32>), grid, block, 0, s, a);
-            else hipLaunchKernelGGL((k_gemm<false, 32>), grid, block, 0, s, a);
-        }
+        if (bn == 128) hipLaunchKernelGGL((k_gemm<128>), grid, block, 0, s, a);
+        else if (bn == 64) hipLaunchKernelGGL((k_gemm<64>), grid, block, 0, s, a);
+        else hipLaunchKernelGGL((k_gemm<32>), grid, block, 0, s, a);
         return hipGetLastError();
     }
     // matrix-vector: one token a workgroup for a decode step and for Q8 (whose other token counts come here only
@@ -791,7 +1010,7 @@ hipError_t launch_mat_multi(const MatMultiArgs& a0, bool q8, hipStream_t s) {
         // chip)
         MatMultiArgs t{};
         for (int i = 0; i < a0.count; i++) {
-            if (q8 && tok_wins(a0.m[i].rows, f.n) && tok_fits(a0)) {
+            if (q8 && tok_fits(a0) && (tok_wins(a0.m[i]) || !gemm_fits(f))) {
                 t.m[t.count++] = a0.m[i];
             } else if (const hipError_t e = launch_mat(a0.m[i], q8, s); e != hipSuccess) {
                 return e;

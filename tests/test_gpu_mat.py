@@ -318,6 +318,28 @@ def test_token_tile_kernel(qw, oracle, rows, cols, n):
     ctx.close()
 
 
+# The Q8 GEMM's tiles (256 x 128, 128 x 128, 128 x 64 rows x tokens), partial in rows and tokens, column counts
+# that end in half a step, and one block alone
+@pytest.mark.parametrize("rows,cols,n", [(8150, 96, 1020), (8192, 32, 1024), (8192, 320, 1024), (8000, 96, 1030),
+                                         (4000, 160, 1000), (2040, 96, 1000), (2048, 2080, 990)], ids=lambda v: str(v))
+@pytest.mark.parametrize("post", [0, 1])
+def test_gemm_q8_tiles(qw, oracle, rows, cols, n, post):
+    print(f"gemm q8 tiles {rows}x{cols} n={n} post={post}", flush=True)
+    blocks, _, _ = q8_blocks(114 + rows + n, rows, cols)
+    w8, s = qw.q8_unpack(blocks, rows, cols)
+    x = np.random.default_rng(115 + n).standard_normal((n, cols + 4)).astype(np.float32)
+    x[:, cols:] = np.nan  # past the columns: never read into a product
+    ctx = _ctx(qw)
+    y = torch.full((n + 1, rows + 3), 7.0, device=DEV)
+    ctx.mat(dev(x)[:, :cols], y[:n, :rows], dev(w8), dev(s), post=post, post_scale=0.37)
+    torch.cuda.synchronize()
+    got = y.cpu().numpy()
+    want = oracle.mat(x[:, :cols], w8=w8, s=s, **({"post": 1, "post_scale": 0.37} if post else {}))
+    _check(got[:n, :rows], want, np.abs(w8.astype(np.float32) * np.repeat(s, 32, axis=1)), x[:, :cols])
+    assert np.all(got[n] == 7.0) and np.all(got[:, rows:] == 7.0)
+    ctx.close()
+
+
 @pytest.mark.parametrize("n", [3, 7, 12])
 def test_token_tile_infinities(qw, n):
     """Infinite and NaN inputs below 16 tokens reach the outputs as fp32 products would have them, and only their
