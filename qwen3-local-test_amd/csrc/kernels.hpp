@@ -106,7 +106,9 @@ struct PrefillArgs {
     float eps;
     const unsigned* kbits;  // QSA: per-token key visibility bits [n][kb_words] (nullptr: dense)
     int kb_words;
+    int list;             // filled by launch_prefill
 };
+constexpr int kPfListTiles = 4096;  // QSA prefill: 64-key tiles whose visible ones are listed in LDS, at most
 // Rope widths the prefill kernel's in-kernel query normalization handles: the rotate-half partner of a
 // lane's dim is then in the same lane.
 __host__ __device__ constexpr bool pf_fused_rope_ok(int R, int D) {

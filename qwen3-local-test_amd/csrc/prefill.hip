@@ -33,6 +33,11 @@
 //    the long prefix's last P.V and merge, so its second segment starts without a load round trip.
 //    Launches small enough that two workgroups per tile fit the CUs split every tile's keys in two
 //    instead (same merge), so chunks of up to ~1,024 tokens still fill the chip.
+//  - QSA (key visibility bits): a workgroup first lists, in LDS, the key tiles that some token of its query tile
+//    sees (one pass over the tokens' bits, a ballot per 512 tiles), and walks the list instead of the keys; the
+//    schedule's halves are halves of the listed tiles. 512 tokens on 16,384 keys, blocks of 64, a budget of
+//    2,048 keys (32 of 256 blocks a token, half of a block's score shared by the chunk): 226 -> 151 us. Every
+//    score is masked by its bit as before, so the result does not depend on what the list leaves out.
 #include "common.hpp"
 #include "kernels.hpp"
 
@@ -240,9 +245,12 @@ __device__ __forceinline__ int pf_tiles(const PrefillArgs& a, int tok_per_blk, i
 // told the next one's query tile (next_qt >= 0), issues that tile's raw query loads (into `carry`) and
 // the copies of its first two K tiles right after its own loop, so they complete during its last P.V,
 // merge and stores; the second (PRE) starts from them, and from the norm multipliers already in LDS.
+// QSA: [lo, hi) are entries of `list`, the tile's visible key tiles in LDS (next_list: the next segment's); without
+// a list the tiles themselves.
 template <int D, int IN_DT, bool QF, bool QSA, bool PRE>
 __device__ __forceinline__ void pf_segment(const PrefillArgs& a, int kvh, int qt, int lo, int hi, int slot,
-                                           int next_qt, PfQRaw<D, IN_DT>& carry) {
+                                           int next_qt, PfQRaw<D, IN_DT>& carry, const uint16_t* list = nullptr,
+                                           const uint16_t* next_list = nullptr) {
     constexpr bool NEXT = pf_handover(QF, IN_DT) && !PRE;
     static_assert(!PRE || pf_handover(QF, IN_DT), "hand-over only for in-kernel bf16 rows");
     using C = PfCfg<D>;
@@ -276,6 +284,8 @@ __device__ __forceinline__ void pf_segment(const PrefillArgs& a, int kvh, int qt
     const int maxlen = a.pos + a.n;
     // QSA: the key bits of this lane's token for the current 64-key tile (two words), the next tile's
     // loaded once these are applied; words past the row's end read as zero
+    // the key tile of entry i (entries past the list's end: a tile past the keys)
+    auto tile = [&](int i) -> int { return QSA && list ? __builtin_amdgcn_readfirstlane(list[i]) : i; };
     const unsigned* qrow = QSA ? a.kbits + (size_t)(row_ok ? t : 0) * a.kb_words : nullptr;
     unsigned qw0 = 0xFFFFFFFFu, qw1 = 0xFFFFFFFFu;
     auto qsa_words = [&](int kt) __attribute__((always_inline)) {
@@ -402,7 +412,8 @@ __device__ __forceinline__ void pf_segment(const PrefillArgs& a, int kvh, int qt
     // the lane's part of the row sums.
     float corr = 1.f;
     bool any_rescale = false;
-    auto step = [&](auto do_pv, const f16* Kb, const f16* Vb, int kt) __attribute__((always_inline)) {
+    // (en: the tile's entry, k2: the tile two entries on)
+    auto step = [&](auto do_pv, const f16* Kb, const f16* Vb, int en, int kt, int k2) __attribute__((always_inline)) {
         constexpr bool DO_PV = decltype(do_pv)::value;
         constexpr int M1 = NSLOT / 4;                   // max phase: slots [0, M1)
         constexpr int E0 = M1 + 4, NE = NSLOT - E0;  // exponentials: slots [E0, NSLOT)
@@ -425,8 +436,8 @@ __device__ __forceinline__ void pf_segment(const PrefillArgs& a, int kvh, int qt
             // Past the last tile they read zeros (range-checked) or unused blocks into free buffers.
             if constexpr (i % 6 == 0 && i / 6 < 2 * LOADS) {
                 constexpr int j = i / 6;
-                if constexpr (j < LOADS) copy_piece(rk, sK(kt & 1), kt + 2, j);
-                else copy_piece(rv, sV(kt & 1), kt, j - LOADS);
+                if constexpr (j < LOADS) copy_piece(rk, sK(en & 1), k2, j);
+                else copy_piece(rv, sV(en & 1), kt, j - LOADS);
             }
             if constexpr (slot_issues(NSLOT, DO_PV, i)) {
                 constexpr int u = slot_rank(NSLOT, DO_PV, i);
@@ -491,8 +502,9 @@ __device__ __forceinline__ void pf_segment(const PrefillArgs& a, int kvh, int qt
     // (tile lo + 1 even past hi: the buffer is free and the copy reads zeros or unused blocks, and a
     // fixed number of copies lets the query's loads be waited for without waiting for any copy)
     if constexpr (!PRE) {
-        copy_tile(rk, sK(lo & 1), lo);
-        copy_tile(rk, sK((lo + 1) & 1), lo + 1);
+        const int e0 = tile(lo), e1 = tile(lo + 1);  // (read before a copy is in flight)
+        copy_tile(rk, sK(lo & 1), e0);
+        copy_tile(rk, sK((lo + 1) & 1), e1);
     }
     {
         // the Q^T operand, while the copies fly (the query loads were issued before them). sW is free:
@@ -519,7 +531,10 @@ __device__ __forceinline__ void pf_segment(const PrefillArgs& a, int kvh, int qt
 
     // one tile iteration; the first (QK^T only, no P.V) is peeled off by hand so that the loop body is
     // the full step alone
-    auto iter = [&](auto do_pv, int kt) __attribute__((always_inline)) {
+    // the tiles of the entry at hand, the one before and the two after it (read from the list an iteration ahead,
+    // behind the barrier: no copy is in flight there)
+    int kp = 0, kt = tile(lo), k1 = tile(lo + 1), k2 = tile(lo + 2);
+    auto iter = [&](auto do_pv, int en) __attribute__((always_inline)) {
         constexpr bool DO_PV = decltype(do_pv)::value;
 #pragma unroll
         for (int cq = 0; cq < 4; cq++) sc[cq] = sn[cq];
@@ -527,8 +542,9 @@ __device__ __forceinline__ void pf_segment(const PrefillArgs& a, int kvh, int qt
         // with the buffers this iteration's copies overwrite (K tile kt, V tile kt-2)
         __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0)
         __syncthreads();
-        if (DO_PV && kt * PF_KT > maxlen) {
-            zero_tail(sV((kt - 1) & 1), kt - 1);
+        const int k3 = QSA ? tile(en + 3) : en + 3;
+        if (DO_PV && (kp + 1) * PF_KT > maxlen) {
+            zero_tail(sV((en - 1) & 1), kp);
             __syncthreads();
         }
         const int k0 = kt * PF_KT;
@@ -540,7 +556,7 @@ __device__ __forceinline__ void pf_segment(const PrefillArgs& a, int kvh, int qt
 #pragma unroll
                 for (int j = 0; j < 4; j++)
                     sc[cq][j] = ((((cq >> 1) ? qw1 : qw0) >> (8 * g + 4 * (cq & 1) + j)) & 1u) ? sc[cq][j] : kNegInf;
-            qsa_words(kt + 1);
+            qsa_words(k1);
         }
         if (k0 + PF_KT > wave_nomask) {
             // causal edge: value i of chain cq = 2 b + s holds key k0 + 32 b + 8 g + 4 s + i, visible to
@@ -551,9 +567,10 @@ __device__ __forceinline__ void pf_segment(const PrefillArgs& a, int kvh, int qt
 #pragma unroll
                 for (int j = 0; j < 4; j++) sc[cq][j] = (32 * (cq >> 1) + 4 * (cq & 1) + j) < lim ? sc[cq][j] : kNegInf;
         }
-        const f16* Kb = sK((kt + 1) & 1) + foff_lane;  // tile kt+1 (stale past the last tile: unused)
-        const f16* Vb = sV((kt + 1) & 1) + foff_lane;  // tile kt-1 (no P.V on the first tile)
-        step(do_pv, Kb, Vb, kt);
+        const f16* Kb = sK((en + 1) & 1) + foff_lane;  // the next tile (stale past the last: unused)
+        const f16* Vb = sV((en + 1) & 1) + foff_lane;  // the tile before (no P.V on the first)
+        step(do_pv, Kb, Vb, en, kt, k2);
+        kp = kt, kt = k1, k1 = k2, k2 = k3;
         if (any_rescale) {
 #pragma unroll
             for (int dt = 0; dt < NDT; dt++) acc[dt] *= corr;
@@ -561,14 +578,14 @@ __device__ __forceinline__ void pf_segment(const PrefillArgs& a, int kvh, int qt
         pprev[0] = pcur[0];
         pprev[1] = pcur[1];
     };
-    qsa_words(lo);
+    qsa_words(kt);
     iter(std::false_type{}, lo);
-    for (int kt = lo + 1; kt < hi; kt++) iter(std::true_type{}, kt);
+    for (int en = lo + 1; en < hi; en++) iter(std::true_type{}, en);
     // ---- P.V of the last tile ----
     __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0)
     __syncthreads();
-    if (hi * PF_KT > maxlen) {
-        zero_tail(sV((hi - 1) & 1), hi - 1);
+    if ((kp + 1) * PF_KT > maxlen) {
+        zero_tail(sV((hi - 1) & 1), kp);
         __syncthreads();
     }
     if constexpr (NEXT) {
@@ -576,9 +593,11 @@ __device__ __forceinline__ void pf_segment(const PrefillArgs& a, int kvh, int qt
         // nothing before the next segment's first barrier reads them)
         if (next_qt >= 0) {
             const int tn = next_qt * tok_per_blk + r / G;
+            const int e0 = QSA && next_list ? __builtin_amdgcn_readfirstlane(next_list[0]) : 0;
+            const int e1 = QSA && next_list ? __builtin_amdgcn_readfirstlane(next_list[1]) : 1;
             carry.load(a, tn < a.n ? tn : 0, h, g);
-            copy_tile(rk, sK(0), 0);
-            copy_tile(rk, sK(1), 1);
+            copy_tile(rk, sK(0), e0);
+            copy_tile(rk, sK(1), e1);
         }
     }
     // the gates of this wave's rows, kept as loaded (bf16 pairs or fp32). Bf16 gates of a whole tile are
@@ -684,6 +703,40 @@ __device__ __forceinline__ void pf_segment(const PrefillArgs& a, int kvh, int qt
     }
 }
 
+// QSA: the key tiles of [0, nt) that some token of query tile qt sees, in order, into list[0, count), count >= 1 (an
+// unseen tile stands in where every key is hidden), then three entries nt (past the keys). Returns count. Called by
+// the whole workgroup before any copy; `cnt` holds 8 words.
+__device__ __forceinline__ int pf_visible(const PrefillArgs& a, int tok_per_blk, int qt, int nt, uint16_t* list, int* cnt) {
+    const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
+    const int t0 = qt * tok_per_blk, t1 = min(a.n, t0 + tok_per_blk);
+    int count = 0;
+    for (int k0 = 0; k0 < nt; k0 += 64 * kPfWaves) {
+        const int kt = k0 + tid;
+        unsigned any = 0u;
+        if (kt < nt) {
+            const unsigned* w = a.kbits + (size_t)t0 * a.kb_words + 2 * kt;
+            const bool two = 2 * kt + 1 < a.kb_words;
+#pragma unroll 8
+            for (int t = t0; t < t1; t++, w += a.kb_words) any |= w[0] | w[two ? 1 : 0];
+        }
+        const unsigned long long seen = __ballot(any != 0u);
+        if (lane == 0) cnt[wave] = (int)__popcll(seen);
+        __syncthreads();
+        int at = count;
+        for (int w = 0; w < kPfWaves; w++) {
+            if (w < wave) at += cnt[w];
+            count += cnt[w];
+        }
+        if (any) list[at + (int)__builtin_amdgcn_mbcnt_hi((unsigned)(seen >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)seen, 0u))] = (uint16_t)kt;
+        __syncthreads();
+    }
+    if (tid == 0 && count == 0) list[0] = 0;
+    count = max(1, count);
+    if (tid < 3) list[count + tid] = (uint16_t)nt;
+    __syncthreads();
+    return count;
+}
+
 // Workgroup j of KV head kvh (blockIdx = j * NKV + kvh). Pair p = j / 2 holds query tiles p (short) and
 // n_qt-1-p (long) with T = nl + ns key tiles: j = 2p runs the long tile over [x, nl), j = 2p+1 its
 // first x tiles, then the short tile, x = max(0, nl - ceil(T/2)). With n_qt odd the last workgroup
@@ -697,16 +750,27 @@ __global__ __launch_bounds__(64 * kPfWaves, 1) void k_prefill(PrefillArgs a) {
     const int np = n_qt / 2;
     // segments (query tile, key tiles [lo, hi), partial slot) of this workgroup, in order
     int q0, lo0, hi0, slot0, q1 = 0, hi1 = 0, nseg = 1;
+    // QSA: tile counts are of the visible tiles, listed in LDS (unless the keys have more tiles than a list holds)
+    extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
+    int* cnt = reinterpret_cast<int*>(smem + 4 * PfCfg<D>::TILEE * 2 + D * sizeof(float));
+    uint16_t* list0 = reinterpret_cast<uint16_t*>(cnt + kPfWaves);
+    uint16_t* list1 = list0 + a.list;
+    const bool listed = QSA && a.list > 0;
+    auto tiles = [&](int qt, uint16_t* list) {
+        const int nt = pf_tiles(a, tok_per_blk, qt);
+        return listed ? pf_visible(a, tok_per_blk, qt, nt, list, cnt) : nt;
+    };
+    const uint16_t *l0 = listed ? list0 : nullptr, *l1 = listed ? list1 : nullptr;
     if (a.split_all) {  // two workgroups per tile, longest tiles first: keys [x, nt) and [0, x)
         const int qt = n_qt - 1 - (j >> 1);
-        const int nt = pf_tiles(a, tok_per_blk, qt), x = nt / 2;
+        const int nt = tiles(qt, list0), x = nt / 2;
         if (x == 0 && (j & 1)) return;  // a one-tile range is not split: the partner runs it whole
         q0 = qt, lo0 = (j & 1) ? 0 : x, hi0 = (j & 1) ? x : nt, slot0 = x > 0 ? kvh * a.slots + qt : -1;
     } else if (j >= 2 * np) {  // the middle tile
-        q0 = np, lo0 = 0, hi0 = pf_tiles(a, tok_per_blk, np), slot0 = -1;
+        q0 = np, lo0 = 0, hi0 = tiles(np, list0), slot0 = -1;
     } else {
         const int p = j >> 1, ql = n_qt - 1 - p;
-        const int nl = pf_tiles(a, tok_per_blk, ql), ns = pf_tiles(a, tok_per_blk, p);
+        const int nl = tiles(ql, list0), ns = tiles(p, list1);
         const int x = max(0, nl - (nl + ns + 1) / 2);
         slot0 = x > 0 ? kvh * a.slots + p : -1;
         if ((j & 1) == 0) {
@@ -714,25 +778,32 @@ __global__ __launch_bounds__(64 * kPfWaves, 1) void k_prefill(PrefillArgs a) {
         } else if (x > 0) {  // the long tile's prefix first: its partial is published long before the partner ends
             q0 = ql, lo0 = 0, hi0 = x, q1 = p, hi1 = ns, nseg = 2;
         } else {
-            q0 = p, lo0 = 0, hi0 = ns;
+            q0 = p, lo0 = 0, hi0 = ns, slot0 = -1;
+            l0 = l1;
         }
     }
     PfQRaw<D, IN_DT> carry;
     if constexpr (pf_handover(QF, IN_DT)) {
         // two call sites: the rows handed over are live only between the first segment's loop and the
         // second's prologue (through one runtime segment loop they would stay live through every tile)
-        pf_segment<D, IN_DT, QF, QSA, false>(a, kvh, q0, lo0, hi0, slot0, nseg == 2 ? q1 : -1, carry);
-        if (nseg == 2) pf_segment<D, IN_DT, QF, QSA, true>(a, kvh, q1, 0, hi1, -1, -1, carry);
+        pf_segment<D, IN_DT, QF, QSA, false>(a, kvh, q0, lo0, hi0, slot0, nseg == 2 ? q1 : -1, carry, l0, l1);
+        if (nseg == 2) pf_segment<D, IN_DT, QF, QSA, true>(a, kvh, q1, 0, hi1, -1, -1, carry, l1);
     } else {
         // one call site, so the segment body exists once in the code object
         for (int s = 0; s < nseg; s++)
-            pf_segment<D, IN_DT, QF, QSA, false>(a, kvh, s ? q1 : q0, s ? 0 : lo0, s ? hi1 : hi0, s ? -1 : slot0, -1, carry);
+            pf_segment<D, IN_DT, QF, QSA, false>(a, kvh, s ? q1 : q0, s ? 0 : lo0, s ? hi1 : hi0, s ? -1 : slot0, -1, carry,
+                                                 s ? l1 : l0);
     }
 }
 
 template <int D>
-static hipError_t launch_pf_d(const PrefillArgs& a, int q_dtype, int in_dtype, hipStream_t s) {
+static hipError_t launch_pf_d(const PrefillArgs& a0, int q_dtype, int in_dtype, hipStream_t s) {
     using C = PfCfg<D>;
+    PrefillArgs a = a0;
+    // entries of a visible-tile list: every key tile and the three after the last; none past what LDS holds
+    // beside the tiles (a context of more than 262,144 keys: every tile is read)
+    const int nt = (a.pos + a.n + PF_KT - 1) / PF_KT;
+    a.list = a.kbits && nt <= kPfListTiles ? (nt + 4) & ~1 : 0;
     const int G = a.NH / a.NKV;
     const int tok = PF_ROWS / G;
     const int n_qt = (a.n + tok - 1) / tok;
@@ -741,7 +812,9 @@ static hipError_t launch_pf_d(const PrefillArgs& a, int q_dtype, int in_dtype, h
         return hipErrorInvalidValue;
     const dim3 grid((a.split_all ? 2 : 1) * n_qt * a.NKV), block(64 * kPfWaves);
     // two buffers of a K and a V tile; with in-kernel query normalization, the D norm multipliers after them
-    const size_t shm = 2 * 2 * (size_t)C::TILEE * 2 + (a.q ? 0 : D * sizeof(float));
+    // (QSA: and the list counters and two lists of visible tiles)
+    const size_t shm = 2 * 2 * (size_t)C::TILEE * 2 +
+                       (a.kbits ? D * sizeof(float) + kPfWaves * 4 + 4 * (size_t)a.list : a.q ? 0 : D * sizeof(float));
     auto go = [&](auto kern) {
         hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, (int)shm);
         if (e != hipSuccess) return e;

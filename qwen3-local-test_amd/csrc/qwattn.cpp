@@ -662,7 +662,7 @@ static int prefill_args(qwattn_ctx* c, const void* q, const void* kcache, const 
     const int split_all = 2 * n_qt * g.n_kv_heads <= c->n_cu ? 1 : 0;
     *a = qw::PrefillArgs{q, (const uint16_t*)kcache, (const uint16_t*)vcache, qg, out, pos, n, g.n_heads,
                          g.n_kv_heads, qw::kLog2eHost / std::sqrt((float)g.head_dim), kv_cap, c->pf_part, c->pf_cnt,
-                         qw::pf_split_slots(n_qt, split_all), split_all, nullptr, nullptr, 0, g.rms_eps};
+                         qw::pf_split_slots(n_qt, split_all), split_all, nullptr, nullptr, 0, g.rms_eps, nullptr, 0, 0};
     if (a->slots > c->pf_slots_per_head) return fail(c, QWATTN_EINVAL, "prefill: %d split slots > %d", a->slots, c->pf_slots_per_head);
     return QWATTN_OK;
 }

@@ -434,6 +434,46 @@ def test_prefill_qsa_all_visible_equals_dense(qw):
     assert torch.equal(out, out2)
 
 
+# Chunks whose query tiles see few of the 64-key tiles: lists of visible tiles with long gaps, none visible before
+# the tail, paired and split schedules, partial last tiles
+@pytest.mark.parametrize("pos,n,dt,cr,density", [(4000, 40, "f32", 64, 0.02), (3990, 70, "bf16", 4, 0.002),
+                                                 (2500, 1200, "bf16", 64, 0.02), (1900, 1111, "f32", 16, 0.01),
+                                                 (777, 200, "bf16", 64, 0.0)], ids=lambda v: str(v))
+def test_prefill_qsa_sparse_tiles(qw, oracle, pos, n, dt, cr, density):
+    test_prefill_qsa_parity(qw, oracle, QWEN3_NEXT, pos, n, dt, cr, density, "prefill")
+
+
+def test_prefill_qsa_past_list_limit(qw):
+    """More key tiles than a list of visible ones holds (over 262,144 keys): every tile is read, and a few visible
+    keys at both ends decide the output (float64 attention over them alone; fp16 weights: 2^-11 of each)."""
+    s, pos, n = QWEN3_NEXT, 262200, 9
+    rows = pos + n
+    cap = capacity(rows)
+    g = torch.Generator(device=DEV)
+    g.manual_seed(5)
+    keys = torch.tensor([0, 63, 64, 130000, 262143, 262144, 262199], device=DEV)
+    kr = torch.zeros((cap, s.NKV, s.D), dtype=torch.float16, device=DEV)
+    vr = torch.zeros_like(kr)
+    kr[keys] = torch.randn((len(keys), s.NKV, s.D), device=DEV, generator=g).half()
+    vr[keys] = torch.randn((len(keys), s.NKV, s.D), device=DEV, generator=g).half()
+    kc, vc = qw.k_block(kr), qw.v_block(vr)
+    q = torch.randn((n, s.NH, s.D), device=DEV, generator=g)
+    qg = torch.randn((n, s.NH, 2 * s.D), device=DEV, generator=g)
+    kbits = torch.zeros((n, (rows + 31) // 32), dtype=torch.int32, device=DEV)
+    for k in keys.tolist():
+        bit = 1 << (k % 32)
+        kbits[:, k // 32] |= bit - (1 << 32) if bit >> 31 else bit
+    ctx = make_ctx(qw, s, max_ctx=cap, max_tokens=n)
+    out = torch.full((n, s.NH, s.D), float("nan"), device=DEV)
+    ctx.attend_prefill_qsa(q, kc, vc, cap, qg, out, pos, n, kbits)
+    ctx.sync_status()
+    kd, vd = (t[keys].double().repeat_interleave(s.G, dim=1) for t in (kr, vr))
+    sc = torch.einsum("thd,khd->thk", q.double(), kd) / s.D ** 0.5
+    ref = torch.einsum("thk,khd->thd", torch.softmax(sc, -1), vd) * torch.sigmoid(qg[..., s.D:].double())
+    assert_rows_parity(host(out), ref.cpu().numpy(), "past the list limit")
+    ctx.close()
+
+
 def test_layer_attention_qsa(qw, oracle):
     """qwattn_layer_attention_qsa over a prefill chunk, a 4-token verify pass and a decode step of one layer
     slot, each with its own key bits, against the oracle's masked attention on the cache it built."""
