@@ -94,10 +94,11 @@ struct PrefillArgs {
     int pos, n, NH, NKV;
     float q_scale;
     int cap;              // capacity (positions) of the caches kc, vc
-    float* part;          // [NKV][slots][2 halves][kPfWaves][pf_part_floats(D)]: partials of split query tiles
+    float* part;          // [NKV][slots][parts][kPfWaves][pf_part_floats(D)]: partials of split query tiles
     int* cnt;             // [NKV][slots][kPfWaves] arrival counters, zero between launches
     int slots;            // split tiles per KV head: pf_split_slots(n_qt, split_all)
-    int split_all;        // 0: short and long tiles paired; 1: every tile's keys split over two workgroups
+    int split_all;        // 0: short and long tiles paired (two parts a long tile); else the parts, a workgroup
+                          // each, of every tile's keys
     // queries normalized in the kernel (q == NULL): RMSNorm weights, rope table [>= pos+n][R/2][2], R
     // a multiple of 32 with R/32 in {1, 2, 4, 8} and R <= D (pf_fused_rope_ok), or 0
     const float* qn;
@@ -116,6 +117,16 @@ __host__ __device__ constexpr bool pf_fused_rope_ok(int R, int D) {
 }
 // Split slots per KV head of a launch with n_qt query tiles per KV head.
 __host__ __device__ constexpr int pf_split_slots(int n_qt, int split_all) { return split_all ? n_qt : n_qt / 2; }
+// Parts of a tile's keys when every tile is split: the most that the CUs take at once, up to 16, while a part of
+// the longest tile (nt key tiles, 1.9 us each) keeps as many key tiles as there are parts to merge (1-2 us each):
+// 256 tokens on 8,192 keys (132 tiles) 68.8 us in eight parts, 77.9 in four; 57 on 26,934 (421) 84 in sixteen, 105
+// in eight. From 48 tiles on: 512 tokens on 2,048 (40) 54.3 in two, 55.6 in four. 0 when two do not fit.
+inline int pf_parts(int n_qt, int nkv, int n_cu, int nt) {
+    if (2 * n_qt * nkv > n_cu) return 0;
+    int p = 2;
+    while (p < 16 && 2 * p * n_qt * nkv <= n_cu && nt >= 48 && 4 * p * p <= nt) p *= 2;
+    return p;
+}
 // Waves of a prefill workgroup (16 query rows each).
 constexpr int kPfWaves = 8;
 // Floats of one wave's prefill partial: 64 lanes x (D/4 accumulator values + max and sum).

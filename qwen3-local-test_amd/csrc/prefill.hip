@@ -31,8 +31,11 @@
 //    arrival counters, log-sum-exp merge of the stored partial), so no workgroup ever waits on another.
 //    The workgroup with two segments loads the short tile's query rows and first two K tiles during
 //    the long prefix's last P.V and merge, so its second segment starts without a load round trip.
-//    Launches small enough that two workgroups per tile fit the CUs split every tile's keys in two
-//    instead (same merge), so chunks of up to ~1,024 tokens still fill the chip.
+//    Launches small enough that two workgroups per tile fit the CUs split every tile's keys instead, over
+//    as many workgroups as fit, up to 16 (pf_parts): chunks of up to ~1,024 tokens still fill the chip. The
+//    last wave to arrive merges the parts one after another. Two parts -> as many as fit (fp32 rows, whole
+//    calls): 256 tokens on 8,192 keys 113 -> 69 us, 57 on 26,934 305 -> 84, 40 on 65,496 821 -> 146, 512 on
+//    16,384 209 -> 164.
 //  - QSA (key visibility bits): a workgroup first lists, in LDS, the key tiles that some token of its query tile
 //    sees (one pass over the tokens' bits, a ballot per 512 tiles), and walks the list instead of the keys; the
 //    schedule's halves are halves of the listed tiles. 512 tokens on 16,384 keys, blocks of 64, a budget of
@@ -237,21 +240,21 @@ __device__ __forceinline__ int pf_tiles(const PrefillArgs& a, int tok_per_blk, i
 
 // One segment of a workgroup's schedule: query tile qt (128 rows of KV head kvh) against key tiles
 // [lo, hi). slot < 0: the tile's whole key range; the normalized, gated rows go to the output.
-// slot >= 0: one of the two halves of a split tile. Each wave stores its unnormalized partial
-// (accumulator, reference max, sum) in its half's region of the pair's slot and counts its arrival,
-// unless the partner wave has already arrived; the wave that arrives second merges the two (in a fixed
-// order) and writes the rows, then clears the counter for the next launch.
+// slot >= 0: part `own` (in key order) of the `parts` parts of a split tile. Each wave stores its unnormalized
+// partial (accumulator, reference max, sum) in its part's region of the slot and counts its arrival (of two parts
+// the second to arrive keeps its own); the last to arrive clears the counter for the next launch, merges the parts
+// in a fixed order and writes the rows.
 // Hand-over between a workgroup's two segments (bf16 rows normalized in the kernel): the first segment,
 // told the next one's query tile (next_qt >= 0), issues that tile's raw query loads (into `carry`) and
 // the copies of its first two K tiles right after its own loop, so they complete during its last P.V,
 // merge and stores; the second (PRE) starts from them, and from the norm multipliers already in LDS.
 // QSA: [lo, hi) are entries of `list`, the tile's visible key tiles in LDS (next_list: the next segment's); without
 // a list the tiles themselves.
-template <int D, int IN_DT, bool QF, bool QSA, bool PRE>
+template <int D, int IN_DT, bool QF, bool QSA, bool SPLIT, bool PRE>
 __device__ __forceinline__ void pf_segment(const PrefillArgs& a, int kvh, int qt, int lo, int hi, int slot,
-                                           int next_qt, PfQRaw<D, IN_DT>& carry, const uint16_t* list = nullptr,
-                                           const uint16_t* next_list = nullptr) {
-    constexpr bool NEXT = pf_handover(QF, IN_DT) && !PRE;
+                                           int own, int parts, int next_qt, PfQRaw<D, IN_DT>& carry,
+                                           const uint16_t* list, const uint16_t* next_list = nullptr) {
+    constexpr bool NEXT = !SPLIT && pf_handover(QF, IN_DT) && !PRE;
     static_assert(!PRE || pf_handover(QF, IN_DT), "hand-over only for in-kernel bf16 rows");
     using C = PfCfg<D>;
     constexpr int NKS = C::NKS, NDT = C::NDT, BLKE = C::BLKE, TILEE = C::TILEE, LOADS = C::LOADS;
@@ -632,20 +635,21 @@ __device__ __forceinline__ void pf_segment(const PrefillArgs& a, int kvh, int qt
         l_run = __uint_as_float(sx[0]) + __uint_as_float(sx[1]);
     }
     if (slot >= 0) {
-        // a wave's partial: accumulator dim tile dt of every lane as 1 KB, then (max, sum) per lane;
-        // each half of the tile has its own region (half 1: keys from lo > 0) and reads the other's
+        // a wave's partial: accumulator dim tile dt of every lane as 1 KB, then (max, sum) per lane; each part of
+        // the tile has its own region
         constexpr int PSTR = pf_part_floats(D);
-        const int own = lo > 0 ? 1 : 0;
-        float* pw = a.part + (((size_t)slot * 2 + own) * kPfWaves + wave) * PSTR;
-        float* pr = a.part + (((size_t)slot * 2 + (1 - own)) * kPfWaves + wave) * PSTR;
+        auto region = [&](int part) {
+            return __builtin_amdgcn_make_buffer_rsrc(a.part + (((size_t)slot * parts + part) * kPfWaves + wave) * PSTR,
+                                                     (short)0, PSTR * 4, 0x00020000);
+        };
         int* cw = a.cnt + slot * kPfWaves + wave;
-        const __amdgpu_buffer_rsrc_t rp = __builtin_amdgcn_make_buffer_rsrc(pw, (short)0, PSTR * 4, 0x00020000);
-        const __amdgpu_buffer_rsrc_t rq = __builtin_amdgcn_make_buffer_rsrc(pr, (short)0, PSTR * 4, 0x00020000);
         const float mu = m_run == kNegInf ? 0.f : m_run;  // the offset the weights were taken against
-        int other = __builtin_amdgcn_readfirstlane(__hip_atomic_load(cw, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
-        if (other == 0) {
-            // first (as far as this wave can tell): publish the partial (device-coherent stores,
-            // acknowledged before the arrival is counted), then count
+        // of two parts the second wave to arrive need not store its own
+        if constexpr (!SPLIT) parts = 2;
+        int others = parts > 2 ? 0 : __builtin_amdgcn_readfirstlane(__hip_atomic_load(cw, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
+        if (others == 0) {
+            // publish the partial (device-coherent stores, acknowledged before the arrival is counted), then count
+            const __amdgpu_buffer_rsrc_t rp = region(own);
 #pragma unroll
             for (int dt = 0; dt < NDT; dt++) __builtin_amdgcn_raw_buffer_store_b128(acc[dt], rp, (dt * 64 + lane) * 16, 0, kScDevice);
             __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(u32x2_t, f32x2{mu, l_run}), rp,
@@ -653,41 +657,75 @@ __device__ __forceinline__ void pf_segment(const PrefillArgs& a, int kvh, int qt
             __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0)
             int old = 0;
             if (lane == 0) old = __hip_atomic_fetch_add(cw, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            other = __builtin_amdgcn_readfirstlane(old);
-            if (other == 0) return;  // the partner wave merges
+            others = __builtin_amdgcn_readfirstlane(old);
+            if (others < parts - 1) return;  // a later one merges
         }
-        // the partner's loads stay behind the count that says its partial is complete
+        // the other parts' loads stay behind the count that says their partials are complete
         asm volatile("" ::: "memory");
-        // second: the partner's partial (published before its count) merged into this wave's, one dim
-        // tile at a time with two more in flight (the whole partial in registers at once would spill)
-        const f32x2 ml2 = __builtin_bit_cast(f32x2, __builtin_amdgcn_raw_buffer_load_b64(rq, NDT * 64 * 16 + lane * 8, 0, kScDevice));
-        constexpr int NB = NDT < 6 ? NDT : 6;
-        f32x4 o2[NB];
-        auto load_dt = [&](int dt) __attribute__((always_inline)) {
-            o2[dt % NB] = __builtin_amdgcn_raw_buffer_load_b128(rq, (dt * 64 + lane) * 16, 0, kScDevice);
-        };
-        static_for<0, NB - 1>([&](auto ic) __attribute__((always_inline)) { load_dt(ic.value); });
         if (lane == 0) __hip_atomic_store(cw, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        // fixed order whichever wave merges: the key-suffix half (lo > 0) is the first term, so the
-        // result does not depend on arrival order
-        const bool own_first = own == 1;
-        const float muf = own_first ? mu : ml2[0], mus = own_first ? ml2[0] : mu;
-        const float lf = own_first ? l_run : ml2[1], ls = own_first ? ml2[1] : l_run;
-        const bool vf = lf > 0.f, vs = ls > 0.f;
-        const float mx = vf ? (vs ? fmaxf(muf, mus) : muf) : mus;
-        const float cf = vf ? exp2_fast(muf - mx) : 0.f, cs = vs ? exp2_fast(mus - mx) : 0.f;
-        l_run = __builtin_fmaf(ls, cs, lf * cf);
-        static_for<0, NDT>([&](auto ic) __attribute__((always_inline)) {
-            constexpr int dt = decltype(ic)::value;
-            if constexpr (dt + NB - 1 < NDT) load_dt(dt + NB - 1);
-            __builtin_amdgcn_sched_barrier(0);
+        if (!SPLIT || parts == 2) {
+            // second: the partner's partial (published before its count) merged into this wave's, one dim
+            // tile at a time with two more in flight (the whole partial in registers at once would spill)
+            const __amdgpu_buffer_rsrc_t rq = region(1 - own);
+            const f32x2 ml2 = __builtin_bit_cast(f32x2, __builtin_amdgcn_raw_buffer_load_b64(rq, NDT * 64 * 16 + lane * 8, 0, kScDevice));
+            constexpr int NB = NDT < 6 ? NDT : 6;
+            f32x4 o2[NB];
+            auto load_dt = [&](int dt) __attribute__((always_inline)) {
+                o2[dt % NB] = __builtin_amdgcn_raw_buffer_load_b128(rq, (dt * 64 + lane) * 16, 0, kScDevice);
+            };
+            static_for<0, NB - 1>([&](auto ic) __attribute__((always_inline)) { load_dt(ic.value); });
+            // fixed order whichever wave merges: the key-suffix half (lo > 0) is the first term, so the
+            // result does not depend on arrival order
+            const bool own_first = own == 1;
+            const float muf = own_first ? mu : ml2[0], mus = own_first ? ml2[0] : mu;
+            const float lf = own_first ? l_run : ml2[1], ls = own_first ? ml2[1] : l_run;
+            const bool vf = lf > 0.f, vs = ls > 0.f;
+            const float mx = vf ? (vs ? fmaxf(muf, mus) : muf) : mus;
+            const float cf = vf ? exp2_fast(muf - mx) : 0.f, cs = vs ? exp2_fast(mus - mx) : 0.f;
+            l_run = __builtin_fmaf(ls, cs, lf * cf);
+            static_for<0, NDT>([&](auto ic) __attribute__((always_inline)) {
+                constexpr int dt = decltype(ic)::value;
+                if constexpr (dt + NB - 1 < NDT) load_dt(dt + NB - 1);
+                __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-            for (int i = 0; i < 4; i++) {
-                const float x = acc[dt][i], y = o2[dt % NB][i];
-                acc[dt][i] = __builtin_fmaf(own_first ? y : x, cs, (own_first ? x : y) * cf);
+                for (int i = 0; i < 4; i++) {
+                    const float x = acc[dt][i], y = o2[dt % NB][i];
+                    acc[dt][i] = __builtin_fmaf(own_first ? y : x, cs, (own_first ? x : y) * cf);
+                }
+                __builtin_amdgcn_sched_barrier(0);
+            });
+        } else {
+            // every part, this wave's own among them, from the last keys to the first, one dim tile at a time with
+            // a few more in flight: the result does not depend on which wave came last
+            float rm = 0.f, rl = 0.f;
+#pragma unroll
+            for (int dt = 0; dt < NDT; dt++) acc[dt] = f32x4{};
+#pragma unroll 1
+            for (int part = parts - 1; part >= 0; part--) {
+                const __amdgpu_buffer_rsrc_t rq = region(part);
+                const f32x2 ml = __builtin_bit_cast(f32x2, __builtin_amdgcn_raw_buffer_load_b64(rq, NDT * 64 * 16 + lane * 8, 0, kScDevice));
+                constexpr int NB = NDT < 6 ? NDT : 6;
+                f32x4 o2[NB];
+                auto load_dt = [&](int dt) __attribute__((always_inline)) {
+                    o2[dt % NB] = __builtin_amdgcn_raw_buffer_load_b128(rq, (dt * 64 + lane) * 16, 0, kScDevice);
+                };
+                static_for<0, NB - 1>([&](auto ic) __attribute__((always_inline)) { load_dt(ic.value); });
+                const bool vf = rl > 0.f, vs = ml[1] > 0.f;
+                const float mx = vf ? (vs ? fmaxf(rm, ml[0]) : rm) : ml[0];
+                const float cf = vf ? exp2_fast(rm - mx) : 0.f, cs = vs ? exp2_fast(ml[0] - mx) : 0.f;
+                rl = __builtin_fmaf(ml[1], cs, rl * cf);
+                rm = mx;
+                static_for<0, NDT>([&](auto ic) __attribute__((always_inline)) {
+                    constexpr int dt = decltype(ic)::value;
+                    if constexpr (dt + NB - 1 < NDT) load_dt(dt + NB - 1);
+                    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                    for (int i = 0; i < 4; i++) acc[dt][i] = __builtin_fmaf(o2[dt % NB][i], cs, acc[dt][i] * cf);
+                    __builtin_amdgcn_sched_barrier(0);
+                });
             }
-            __builtin_amdgcn_sched_barrier(0);
-        });
+            l_run = rl;
+        }
     }
     if (!kGateEarly || slot >= 0) load_gates();
     if (row_ok) {
@@ -741,7 +779,8 @@ __device__ __forceinline__ int pf_visible(const PrefillArgs& a, int tok_per_blk,
 // n_qt-1-p (long) with T = nl + ns key tiles: j = 2p runs the long tile over [x, nl), j = 2p+1 its
 // first x tiles, then the short tile, x = max(0, nl - ceil(T/2)). With n_qt odd the last workgroup
 // runs the middle tile alone.
-template <int D, int IN_DT, bool QF, bool QSA>
+// SPLIT: the split schedule (a.split_all parts, a power of two, a workgroup each), else the paired one.
+template <int D, int IN_DT, bool QF, bool QSA, bool SPLIT>
 __global__ __launch_bounds__(64 * kPfWaves, 1) void k_prefill(PrefillArgs a) {
     const int G = a.NH / a.NKV;
     const int tok_per_blk = PF_ROWS / G;
@@ -749,7 +788,7 @@ __global__ __launch_bounds__(64 * kPfWaves, 1) void k_prefill(PrefillArgs a) {
     const int kvh = blockIdx.x % a.NKV, j = blockIdx.x / a.NKV;
     const int np = n_qt / 2;
     // segments (query tile, key tiles [lo, hi), partial slot) of this workgroup, in order
-    int q0, lo0, hi0, slot0, q1 = 0, hi1 = 0, nseg = 1;
+    int q0, lo0, hi0, slot0, own0 = 0, parts0 = 2, q1 = 0, hi1 = 0, nseg = 1;
     // QSA: tile counts are of the visible tiles, listed in LDS (unless the keys have more tiles than a list holds)
     extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
     int* cnt = reinterpret_cast<int*>(smem + 4 * PfCfg<D>::TILEE * 2 + D * sizeof(float));
@@ -761,11 +800,16 @@ __global__ __launch_bounds__(64 * kPfWaves, 1) void k_prefill(PrefillArgs a) {
         return listed ? pf_visible(a, tok_per_blk, qt, nt, list, cnt) : nt;
     };
     const uint16_t *l0 = listed ? list0 : nullptr, *l1 = listed ? list1 : nullptr;
-    if (a.split_all) {  // two workgroups per tile, longest tiles first: keys [x, nt) and [0, x)
-        const int qt = n_qt - 1 - (j >> 1);
-        const int nt = tiles(qt, list0), x = nt / 2;
-        if (x == 0 && (j & 1)) return;  // a one-tile range is not split: the partner runs it whole
-        q0 = qt, lo0 = (j & 1) ? 0 : x, hi0 = (j & 1) ? x : nt, slot0 = x > 0 ? kvh * a.slots + qt : -1;
+    if constexpr (SPLIT) {  // longest tiles first, an equal run of key tiles each
+        const int lg = __builtin_ctz((unsigned)a.split_all);
+        const int qt = n_qt - 1 - (j >> lg), part = a.split_all - 1 - (j & (a.split_all - 1));
+        const int nt = tiles(qt, list0);
+        parts0 = min(a.split_all, nt);  // a part holds a tile at least
+        if (part >= parts0) return;
+        q0 = qt, own0 = part;
+        lo0 = nt < a.split_all ? part : nt * part >> lg;
+        hi0 = nt < a.split_all ? part + 1 : nt * (part + 1) >> lg;
+        slot0 = parts0 > 1 ? kvh * a.slots + qt : -1;
     } else if (j >= 2 * np) {  // the middle tile
         q0 = np, lo0 = 0, hi0 = tiles(np, list0), slot0 = -1;
     } else {
@@ -774,7 +818,7 @@ __global__ __launch_bounds__(64 * kPfWaves, 1) void k_prefill(PrefillArgs a) {
         const int x = max(0, nl - (nl + ns + 1) / 2);
         slot0 = x > 0 ? kvh * a.slots + p : -1;
         if ((j & 1) == 0) {
-            q0 = ql, lo0 = x, hi0 = nl;
+            q0 = ql, lo0 = x, hi0 = nl, own0 = 1;
         } else if (x > 0) {  // the long tile's prefix first: its partial is published long before the partner ends
             q0 = ql, lo0 = 0, hi0 = x, q1 = p, hi1 = ns, nseg = 2;
         } else {
@@ -783,16 +827,18 @@ __global__ __launch_bounds__(64 * kPfWaves, 1) void k_prefill(PrefillArgs a) {
         }
     }
     PfQRaw<D, IN_DT> carry;
-    if constexpr (pf_handover(QF, IN_DT)) {
+    if constexpr (SPLIT) {
+        pf_segment<D, IN_DT, QF, QSA, true, false>(a, kvh, q0, lo0, hi0, slot0, own0, parts0, -1, carry, l0);
+    } else if constexpr (pf_handover(QF, IN_DT)) {
         // two call sites: the rows handed over are live only between the first segment's loop and the
         // second's prologue (through one runtime segment loop they would stay live through every tile)
-        pf_segment<D, IN_DT, QF, QSA, false>(a, kvh, q0, lo0, hi0, slot0, nseg == 2 ? q1 : -1, carry, l0, l1);
-        if (nseg == 2) pf_segment<D, IN_DT, QF, QSA, true>(a, kvh, q1, 0, hi1, -1, -1, carry, l1);
+        pf_segment<D, IN_DT, QF, QSA, SPLIT, false>(a, kvh, q0, lo0, hi0, slot0, own0, parts0, nseg == 2 ? q1 : -1, carry, l0, l1);
+        if (nseg == 2) pf_segment<D, IN_DT, QF, QSA, SPLIT, true>(a, kvh, q1, 0, hi1, -1, 0, 0, -1, carry, l1);
     } else {
         // one call site, so the segment body exists once in the code object
         for (int s = 0; s < nseg; s++)
-            pf_segment<D, IN_DT, QF, QSA, false>(a, kvh, s ? q1 : q0, s ? 0 : lo0, s ? hi1 : hi0, s ? -1 : slot0, -1, carry,
-                                                 s ? l1 : l0);
+            pf_segment<D, IN_DT, QF, QSA, SPLIT, false>(a, kvh, s ? q1 : q0, s ? 0 : lo0, s ? hi1 : hi0, s ? -1 : slot0, own0, parts0,
+                                                 -1, carry, s ? l1 : l0);
     }
 }
 
@@ -810,7 +856,7 @@ static hipError_t launch_pf_d(const PrefillArgs& a0, int q_dtype, int in_dtype, 
     // the split tiles' partial slots and counters are the caller's (sized for `slots` per KV head)
     if (a.n < 1 || a.slots != pf_split_slots(n_qt, a.split_all) || (a.slots > 0 && (!a.part || !a.cnt)))
         return hipErrorInvalidValue;
-    const dim3 grid((a.split_all ? 2 : 1) * n_qt * a.NKV), block(64 * kPfWaves);
+    const dim3 grid((a.split_all ? a.split_all : 1) * n_qt * a.NKV), block(64 * kPfWaves);
     // two buffers of a K and a V tile; with in-kernel query normalization, the D norm multipliers after them
     // (QSA: and the list counters and two lists of visible tiles)
     const size_t shm = 2 * 2 * (size_t)C::TILEE * 2 +
@@ -823,14 +869,17 @@ static hipError_t launch_pf_d(const PrefillArgs& a0, int q_dtype, int in_dtype, 
     };
     // fp32 queries reach this kernel converted to the fp16 operand (launch_q_f16); without q the kernel
     // normalizes the query half of qg itself
-    if (q_dtype != 2) return hipErrorInvalidValue;
+    if (q_dtype != 2 || (a.split_all & (a.split_all - 1))) return hipErrorInvalidValue;
+    auto pick = [&](auto qf, auto qsa) {
+        constexpr bool QF = decltype(qf)::value, QSA = decltype(qsa)::value;
+        if (a.split_all) return in_dtype == 0 ? go(k_prefill<D, 0, QF, QSA, true>) : go(k_prefill<D, 1, QF, QSA, true>);
+        return in_dtype == 0 ? go(k_prefill<D, 0, QF, QSA, false>) : go(k_prefill<D, 1, QF, QSA, false>);
+    };
     if (!a.q) {
         if (!a.qn || (a.R && !a.rope) || !pf_fused_rope_ok(a.R, D)) return hipErrorInvalidValue;
-        if (a.kbits) return in_dtype == 0 ? go(k_prefill<D, 0, true, true>) : go(k_prefill<D, 1, true, true>);
-        return in_dtype == 0 ? go(k_prefill<D, 0, true, false>) : go(k_prefill<D, 1, true, false>);
+        return a.kbits ? pick(std::true_type{}, std::true_type{}) : pick(std::true_type{}, std::false_type{});
     }
-    if (a.kbits) return in_dtype == 0 ? go(k_prefill<D, 0, false, true>) : go(k_prefill<D, 1, false, true>);
-    return in_dtype == 0 ? go(k_prefill<D, 0, false, false>) : go(k_prefill<D, 1, false, false>);
+    return a.kbits ? pick(std::false_type{}, std::true_type{}) : pick(std::false_type{}, std::false_type{});
 }
 
 // fp16(q * scale): the prefill operand from fp32 queries; n4 groups of 4 values

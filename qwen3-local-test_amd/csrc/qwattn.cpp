@@ -33,7 +33,8 @@ struct qwattn_ctx {
     void* q16 = nullptr;         // [max_tokens][NH][D] layer-path query (fp16, pre-scaled)
     float* pf_part = nullptr;    // prefill: partials of split query tiles (qw::PrefillArgs::part)
     int* pf_cnt = nullptr;       // prefill: their arrival counters, zero between launches
-    int pf_slots_per_head = 0;   // prefill: split slots per KV head in pf_part / pf_cnt
+    int pf_slots_per_head = 0;   // prefill: split slots per KV head in pf_cnt
+    int pf_parts_per_head = 0;   // prefill: split tiles' parts per KV head in pf_part
     float* qsa_scores = nullptr; // QSA select: block scores of the tokens of one launch (kQsaScoreBytes)
     int* qsa_cnt = nullptr;      // QSA select: per-token arrival counters [max_tokens], zero between launches
     unsigned* qsa_hist = nullptr; // QSA select: first-digit histograms [qsa_hist_n][2048], zero between launches
@@ -254,13 +255,16 @@ int qwattn_create(qwattn_ctx** out, int device, const qwattn_config* cfg) {
     const size_t qn = (size_t)cfg->max_tokens * NH * D;
     // prefill split slots per KV head: a pair of query tiles each (paired schedule) or a tile each (split
     // schedule, only while two workgroups per tile fit the CUs), at least one so the pointers are never
-    // null; kPfWaves waves each, a partial region per half of the split tile
+    // null; kPfWaves waves each, a partial region per part of a split tile (two of a pair's long tile, up to 16
+    // while the parts' workgroups fit the CUs)
     const int qt_max = qw::pf_query_tiles(cfg->max_tokens, NH / NKV);
     c->pf_slots_per_head = std::max(1, std::max(qt_max / 2, std::min(qt_max, c->n_cu / (2 * NKV))));
+    c->pf_parts_per_head = std::max(2, std::max(qt_max, std::min(16 * qt_max, c->n_cu / NKV)));
     const size_t pf_slots = (size_t)NKV * c->pf_slots_per_head * qw::kPfWaves;
+    const size_t pf_parts = (size_t)NKV * c->pf_parts_per_head * qw::kPfWaves;
     c->qsa_hist_n = std::min(cfg->max_tokens, qw::kQsaHistTokens);
     const size_t hist_tokens = (size_t)c->qsa_hist_n;
-    bool ok = hipMalloc(&c->pf_part, sizeof(float) * 2 * pf_slots * qw::pf_part_floats(D)) == hipSuccess &&
+    bool ok = hipMalloc(&c->pf_part, sizeof(float) * pf_parts * qw::pf_part_floats(D)) == hipSuccess &&
               hipMalloc(&c->pf_cnt, sizeof(int) * pf_slots) == hipSuccess &&
               hipMalloc(&c->inv_freq, sizeof(float) * std::max(1, R / 2)) == hipSuccess &&
               hipMalloc(&c->rope, sizeof(float) * rope_n) == hipSuccess &&
@@ -655,15 +659,15 @@ int qwattn_combine(qwattn_ctx* c, void* stream, const void* qg, int in_dtype, fl
 static int prefill_args(qwattn_ctx* c, const void* q, const void* kcache, const void* vcache, int kv_cap,
                         const void* qg, float* out, int pos, int n, qw::PrefillArgs* a) {
     const qwattn_config& g = c->cfg;
-    // Few query tiles (two workgroups per tile still fit the CUs): every tile's keys are split over two
-    // workgroups; otherwise short and long tiles are paired. Either way the split tiles fit the slots
-    // sized at creation (n <= max_tokens by check_call; split_all only when 2 * n_qt * NKV <= n_cu).
+    // Few query tiles (two workgroups per tile still fit the CUs): every tile's keys are split over two or more
+    // workgroups; otherwise short and long tiles are paired. Either way the split tiles fit the slots and parts
+    // sized at creation (n <= max_tokens by check_call).
     const int n_qt = qw::pf_query_tiles(n, g.n_heads / g.n_kv_heads);
-    const int split_all = 2 * n_qt * g.n_kv_heads <= c->n_cu ? 1 : 0;
+    const int split_all = qw::pf_parts(n_qt, g.n_kv_heads, c->n_cu, (pos + n + 63) / 64);
     *a = qw::PrefillArgs{q, (const uint16_t*)kcache, (const uint16_t*)vcache, qg, out, pos, n, g.n_heads,
                          g.n_kv_heads, qw::kLog2eHost / std::sqrt((float)g.head_dim), kv_cap, c->pf_part, c->pf_cnt,
                          qw::pf_split_slots(n_qt, split_all), split_all, nullptr, nullptr, 0, g.rms_eps, nullptr, 0, 0};
-    if (a->slots > c->pf_slots_per_head) return fail(c, QWATTN_EINVAL, "prefill: %d split slots > %d", a->slots, c->pf_slots_per_head);
+    if (a->slots > c->pf_slots_per_head || a->slots * std::max(2, split_all) > c->pf_parts_per_head) return fail(c, QWATTN_EINVAL, "prefill: %d split slots > %d", a->slots, c->pf_slots_per_head);
     return QWATTN_OK;
 }
 

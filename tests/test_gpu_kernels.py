@@ -537,6 +537,14 @@ def test_prefill_parity(qw, oracle, s, pos, n):
     assert_rows_parity(out, ref, f"{s} pos={pos} n={n}")
 
 
+# Small chunks on long contexts: every tile's keys over 4, 8 and 16 workgroups, and over fewer than asked for where
+# a tile has fewer key tiles
+@pytest.mark.parametrize("s,pos,n", [(QWEN3_NEXT, 1500, 300), (QWEN3_NEXT, 4060, 40), (QWEN3_NEXT, 16411, 37),
+                                     (TINY, 17000, 33), (D128, 5000, 70)], ids=lambda v: repr(v))
+def test_prefill_many_parts(qw, oracle, s, pos, n):
+    test_prefill_parity(qw, oracle, s, pos, n)
+
+
 @pytest.mark.parametrize("s,pos,n", CASES_PF, ids=lambda v: repr(v))
 def test_prefill_entry_parity(qw, oracle, s, pos, n):
     """qwattn_prefill against the oracle and against the two entry points called in sequence (norm/rope/
