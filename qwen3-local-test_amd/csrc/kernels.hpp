@@ -1,12 +1,25 @@
 // Host-side launchers of the gfx950 kernels (internal to libqwattn; the C ABI in qwattn.cpp checks
 // every shape and pointer before calling these). K/V caches use the blocked layout of common.hpp.
 #pragma once
+#include <atomic>
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
 namespace qw {
 
 constexpr float kLog2eHost = 1.4426950408889634f;
+
+// Raises a kernel's dynamic LDS past the default 64 KB, once per device (`raised`: a bit each).
+inline hipError_t raise_lds(const void* kernel, size_t lds, std::atomic<uint64_t>& raised) {
+    if (lds <= 64 * 1024) return hipSuccess;
+    int dev = 0;
+    if (hipGetDevice(&dev) != hipSuccess) return hipErrorInvalidDevice;
+    const uint64_t bit = 1ull << (dev & 63);
+    if (raised.load(std::memory_order_acquire) & bit) return hipSuccess;
+    const hipError_t e = hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+    if (e == hipSuccess) raised.fetch_or(bit, std::memory_order_acq_rel);
+    return e;
+}
 
 struct NormRopeArgs {
     const void* qg;      // [n][NH][2D]
@@ -171,6 +184,10 @@ struct QsaSelectArgs {
     int hcopies;          // histogram copies a token (n * hcopies <= kQsaHistTokens)
 };
 hipError_t launch_qsa_select(const QsaSelectArgs& a, int in_dtype, hipStream_t s);
+// The same for many tokens (from kQsaMany; at most 32,768 complete blocks; raw, cnt, hist and cand unused): scores
+// in one launch, the selections in another.
+hipError_t launch_qsa_select_many(const QsaSelectArgs& a, int in_dtype, hipStream_t s);
+constexpr int kQsaMany = 16, kQsaManyBlocks = 32768;
 // First-digit histograms (2,048 bins) a select launch may use: a token takes 1 to 8 copies
 constexpr int kQsaHistTokens = 1024;
 // The two-launch form (more than 32,768 complete blocks): selection workgroups of kQsaSelBlocks blocks, each

@@ -17,7 +17,6 @@
 // block scale once per group. The partial dot products are summed over the wave with DPP row operations and
 // permlane swaps.
 #include <algorithm>
-#include <atomic>
 
 #include "common.hpp"
 #include "kernels.hpp"
@@ -832,18 +831,6 @@ constexpr size_t gemm_lds() {
 }  // namespace
 
 namespace {
-
-// Raises a kernel's dynamic LDS past the default 64 KB, once per device (`raised`: a bit each).
-hipError_t raise_lds(const void* kernel, size_t lds, std::atomic<uint64_t>& raised) {
-    if (lds <= 64 * 1024) return hipSuccess;
-    int dev = 0;
-    if (hipGetDevice(&dev) != hipSuccess) return hipErrorInvalidDevice;
-    const uint64_t bit = 1ull << (dev & 63);
-    if (raised.load(std::memory_order_acquire) & bit) return hipSuccess;
-    const hipError_t e = hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-    if (e == hipSuccess) raised.fetch_or(bit, std::memory_order_acq_rel);
-    return e;
-}
 
 template <int TT, int R, int NS, int B, int KW>
 hipError_t launch_tok(MatMultiArgs a, hipStream_t s) {

@@ -470,10 +470,14 @@ struct FirstDigit {
     // the bin of the top-th largest key, scanned from the top two bins a thread: s_misc[0] the digit, [1] the
     // keys of larger digits, [2] the bin's keys (every thread reads them after the barrier)
     __device__ __forceinline__ void scan(int top, int* s_misc, int* s_scan) const {
-        const int tid = threadIdx.x;
         unsigned g1 = 0u, g0 = 0u;
 #pragma unroll
         for (int i = 0; i < kQsaHistCopies; i++) g0 += gv[i][0], g1 += gv[i][1];
+        scan_bins(g1, g0, top, s_misc, s_scan);
+    }
+    // ... from this thread's two counts
+    __device__ __forceinline__ void scan_bins(unsigned g1, unsigned g0, int top, int* s_misc, int* s_scan) const {
+        const int tid = threadIdx.x;
         const int larger = block_excl_scan((int)(g1 + g0), s_scan + 32);
         if (larger < top && larger + (int)(g1 + g0) >= top) {  // exactly one thread
             const bool in1 = larger + (int)g1 >= top;
@@ -498,7 +502,8 @@ struct FirstDigit {
 // them held in registers, nblk <= KR * 1,024; KR == 0: read from memory at each use), so that each wave's
 // ballot over one of them is two mask words. A stored word L orders opposite to its key, and as a signed
 // value every L of a block (bit 31 set) lies below the 0 past nblk: key > T is (int) L < (int) ~T.
-template <int KR, bool COH>
+// LOCAL: the histogram is counted here instead, in LDS from the row itself (gh unused).
+template <int KR, bool COH, bool LOCAL = false>
 __device__ __forceinline__ void select_blocks(const QsaSelectArgs& a, __amdgpu_buffer_rsrc_t rs, int t, int nblk,
                                               unsigned* s_mask, int* s_misc, int* s_scan, unsigned* s_hist,
                                               unsigned* s_ck, unsigned* gh, int nh) {
@@ -507,7 +512,8 @@ __device__ __forceinline__ void select_blocks(const QsaSelectArgs& a, __amdgpu_b
     const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
     const int nch = KR > 0 ? KR : (nblk + kQsaThreads - 1) / kQsaThreads;
     unsigned* s_cb = s_ck + kQsaCand;
-    const FirstDigit fd(gh, nh);
+    static_assert(!LOCAL || KR > 0, "the row's keys in registers");
+    const FirstDigit fd(gh, LOCAL ? 0 : nh);
     auto ld = [&](int j) -> unsigned { return __builtin_amdgcn_raw_buffer_load_b32(rs, (j * kQsaThreads + tid) * 4, 0, AUX); };
     unsigned kr[KR > 0 ? KR : 1];
     if constexpr (KR > 0) {
@@ -517,8 +523,19 @@ __device__ __forceinline__ void select_blocks(const QsaSelectArgs& a, __amdgpu_b
     // the later passes' LDS bins start at zero
 #pragma unroll
     for (int i = 0; i < 4; i++) s_hist[tid + i * kQsaThreads] = 0u;
-    fd.scan(a.top, s_misc, s_scan);
-    fd.clear();
+    if constexpr (LOCAL) {
+        s_mask[tid] = 0u, s_mask[tid + kQsaThreads] = 0u;  // the first digit's bins, until the mask is written
+        __syncthreads();
+#pragma unroll
+        for (int j = 0; j < KR; j++)
+            if ((int)kr[j] < 0)  // not past nblk
+                __hip_atomic_fetch_add(&s_mask[~kr[j] >> 20], 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+        __syncthreads();
+        fd.scan_bins(s_mask[2047 - 2 * tid], s_mask[2046 - 2 * tid], a.top, s_misc, s_scan);
+    } else {
+        fd.scan(a.top, s_misc, s_scan);
+        fd.clear();
+    }
     const unsigned d1 = (unsigned)s_misc[0];
     const int need = a.top - s_misc[1], cnt = s_misc[2];  // to take from the bin, of cnt
     if (cnt > kQsaCand) {
@@ -898,6 +915,144 @@ __global__ __launch_bounds__(kQsaThreads) __attribute__((amdgpu_waves_per_eu(4, 
     select_blocks<KR, true>(a, rs, t, nblk, s_mask, s_misc, s_scan, s_hist, s_ck, gh, a.hcopies);  // KR: the last token's
 }
 
+// ---- many tokens: scores on the matrix cores, then a workgroup's selection a token --------------------------
+// Scores of 32 tokens x 128 blocks a workgroup (four waves, 32 blocks each): sum over the heads of
+// relu(q_h . pooled), each product a chain of v_mfma_f32_32x32x2_f32 (fp32 multiply-adds, as the 16-lane dot
+// products of the few-token kernel). A lane (c, h) holds block c's dims [h ID/2, + ID/2) in registers; the tokens'
+// heads are normed and rotated once a workgroup into LDS (rows padded by 16 bytes: their 16-byte reads are free
+// of bank conflicts), 512 head dims at a time. Stored as the few-token kernel stores them: ~score
+// for a token's complete blocks, 0 past them (to the row's end). A token that selects nothing is left out.
+// Bound: the fp32 matrix rate (2.2 GFLOP take 14 us of the chip at 153 TFLOP/s, a large product here), in whole
+// 32 x 32 tiles a wave: 512 tokens x 4,224 blocks of 4 heads x 128 dims (2.06 tiles a SIMD) 43 us; 53 with the rows
+// loaded one at a time. The whole index call there 634 -> 62 us: the few-token kernel normed the query again for
+// every 64 blocks and ran the products on vector units, 16 lanes a key.
+constexpr int kQsaTok = 32, kQsaScoreBlocks = 128;
+constexpr int qsa_score_heads(int ID) { return ID <= 64 ? 8 : ID <= 128 ? 4 : 2; }
+template <int IN_DT, int ID>
+__global__ __launch_bounds__(256) void k_qsa_score(QsaSelectArgs a) {
+    constexpr int HC = qsa_score_heads(ID), ST = ID + 4, DL = ID / 16;  // heads in LDS, row stride, dims a lane
+    __shared__ int s_nblk[kQsaTok];
+    extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
+    float* s_q = reinterpret_cast<float*>(smem);  // [HC][32][ST]
+    const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, c = lane & 31, h = lane >> 5;
+    const int t0 = blockIdx.y * kQsaTok, nt = min(kQsaTok, a.n - t0);
+    const int nlast = (a.pos + t0 + nt) / a.CR;  // the last token's complete blocks: the most of the 32
+    if (nlast <= a.top) return;
+    if (tid < kQsaTok) s_nblk[tid] = (a.pos + t0 + tid + 1) / a.CR;
+    const int b = blockIdx.x * kQsaScoreBlocks + wave * 32 + c;
+    float pk[ID / 2];
+    {
+        const float* row = a.pooled + (size_t)min(b, nlast - 1) * ID + h * (ID / 2);  // past the blocks: not scored
+#pragma unroll
+        for (int i = 0; i < ID / 2; i += 4) {
+            const f32x4 v = *reinterpret_cast<const f32x4*>(row + i);
+            pk[i] = v[0], pk[i + 1] = v[1], pk[i + 2] = v[2], pk[i + 3] = v[3];
+        }
+    }
+    f32x16 sc;
+#pragma unroll
+    for (int j = 0; j < 16; j++) sc[j] = 0.f;
+    const int half = a.R >> 1, grp = tid >> 4, sub = tid & 15;
+    float gm[DL], rp[2][DL][2];  // this lane's gammas, and (cos, sin) of its two tokens (past R: unused)
+#pragma unroll
+    for (int k = 0; k < DL; k++) {
+        const int d = sub + 16 * k, e = d < half ? d : d < a.R ? d - half : 0;
+        gm[k] = a.gamma[d];
+#pragma unroll
+        for (int m = 0; m < 2; m++) {
+            rp[m][k][0] = rp[m][k][1] = 0.f;
+            if (d < a.R) {
+                const float* cs = a.rope + ((size_t)(a.pos + t0 + min(grp + 16 * m, nt - 1)) * half + e) * 2;
+                rp[m][k][0] = cs[0], rp[m][k][1] = cs[1];
+            }
+        }
+    }
+    for (int h0 = 0; h0 < a.IH; h0 += HC) {
+        const int nh = min(HC, a.IH - h0);
+        __syncthreads();
+        // 16 lanes a row (dims sub + 16 k), group grp the tokens grp and grp + 16 of each head: every row loaded
+        // first, then norm and rotation with partners read back from LDS (a row's lanes are in one wave, whose LDS
+        // accesses stay in order)
+        float x[2 * HC][DL];
+#pragma unroll
+        for (int m = 0; m < 2 * HC; m++) {
+            const int tt = min(grp + 16 * (m & 1), nt - 1), hh = min(m >> 1, nh - 1);
+#pragma unroll
+            for (int k = 0; k < DL; k++) x[m][k] = load_in<IN_DT>(a.iq, ((size_t)(t0 + tt) * a.IH + h0 + hh) * ID + sub + 16 * k);
+        }
+#pragma unroll
+        for (int m = 0; m < 2 * HC; m++) {
+            if ((m >> 1) >= nh) break;  // uniform
+            float* row = s_q + ((m >> 1) * kQsaTok + grp + 16 * (m & 1)) * ST;
+            float ss = 0.f;
+#pragma unroll
+            for (int k = 0; k < DL; k++) ss += x[m][k] * x[m][k];
+            ss = sum16(ss);
+            const float r = 1.0f / sqrtf(ss / (float)ID + a.eps);
+#pragma unroll
+            for (int k = 0; k < DL; k++) row[sub + 16 * k] = x[m][k] = x[m][k] * r * gm[k];
+            __builtin_amdgcn_wave_barrier();
+            float y[DL];
+#pragma unroll
+            for (int k = 0; k < DL; k++) {
+                const int d = sub + 16 * k;
+                y[k] = x[m][k];
+                if (d < half) y[k] = x[m][k] * rp[m & 1][k][0] - row[d + half] * rp[m & 1][k][1];
+                else if (d < a.R) y[k] = x[m][k] * rp[m & 1][k][0] + row[d - half] * rp[m & 1][k][1];
+            }
+            __builtin_amdgcn_wave_barrier();
+#pragma unroll
+            for (int k = 0; k < DL; k++) row[sub + 16 * k] = y[k];
+        }
+        __syncthreads();
+        for (int hh = 0; hh < nh; hh++) {
+            const float* q = s_q + (hh * kQsaTok + c) * ST + h * (ID / 2);
+            f32x16 d;
+#pragma unroll
+            for (int j = 0; j < 16; j++) d[j] = 0.f;
+#pragma unroll
+            for (int i = 0; i < ID / 2; i += 4) {
+                const f32x4 v = *reinterpret_cast<const f32x4*>(q + i);
+#pragma unroll
+                for (int k = 0; k < 4; k++) d = __builtin_amdgcn_mfma_f32_32x32x2f32(v[k], pk[i + k], d, 0, 0, 0);
+            }
+#pragma unroll
+            for (int j = 0; j < 16; j++) sc[j] += d[j] > 0.f ? d[j] : 0.f;  // relu; -0 and NaN contribute +0
+        }
+    }
+    if (b >= a.stride) return;
+    // lane (c, h): block c, tokens 8 (j / 4) + 4 h + j % 4
+#pragma unroll
+    for (int j = 0; j < 16; j++) {
+        const int tt = 8 * (j / 4) + 4 * h + j % 4;
+        if (tt >= nt) continue;
+        const int nblk = s_nblk[tt];
+        if (nblk > a.top)
+            reinterpret_cast<unsigned*>(a.scores)[(size_t)(t0 + tt) * a.stride + b] = b < nblk ? ~__float_as_uint(sc[j]) : 0u;
+    }
+}
+
+// Workgroup t selects token t's blocks from its score row.
+template <int KR>
+__global__ __launch_bounds__(kQsaThreads) __attribute__((amdgpu_waves_per_eu(4, 4))) void k_qsa_pick(QsaSelectArgs a) {
+    extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
+    unsigned* s_mask = reinterpret_cast<unsigned*>(smem);
+    int* s_misc = reinterpret_cast<int*>(s_mask + kQsaMaskLds);
+    int* s_scan = s_misc + 32;
+    unsigned* s_hist = reinterpret_cast<unsigned*>(s_scan + 48);
+    const int t = blockIdx.x, nblk = (a.pos + t + 1) / a.CR;
+    if (nblk <= a.top) {
+        if (a.mask)
+            for (int w = threadIdx.x; w < a.mask_words; w += kQsaThreads) a.mask[(size_t)t * a.mask_words + w] = 0xFFFFFFFFu;
+        if (a.kbits)
+            for (int w = threadIdx.x; w < a.kb_words; w += kQsaThreads) a.kbits[(size_t)t * a.kb_words + w] = 0xFFFFFFFFu;
+        return;
+    }
+    const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc(a.scores + (size_t)t * a.stride, (short)0,
+                                                                        a.stride * 4, 0x00020000);
+    select_blocks<KR, false, true>(a, rs, t, nblk, s_mask, s_misc, s_scan, s_hist, s_hist + 4096, nullptr, 0);
+}
+
 // ---- key bits from a block mask (shaders/attention.comp:35-43) -------------------------------------------
 __global__ __launch_bounds__(256) void k_qsa_key_bits(QsaKeyBitsArgs a) {
     const int w = blockIdx.x * 256 + threadIdx.x, t = blockIdx.y;
@@ -942,15 +1097,7 @@ static hipError_t launch_select_kr(const QsaSelectArgs& a, size_t shm, dim3 grid
     static std::atomic<uint64_t> raised{0};  // bit per device
     static const size_t shm_max = qsa_select_lds(1, kQsaMaxHeadDims);
     if (shm > shm_max) return hipErrorInvalidValue;
-    int dev = 0;
-    if (hipGetDevice(&dev) != hipSuccess) return hipErrorInvalidDevice;
-    const uint64_t bit = 1ull << (dev & 63);
-    if (!(raised.load(std::memory_order_acquire) & bit)) {
-        const hipError_t e = hipFuncSetAttribute((const void*)k_qsa_select<IN_DT, KR, MODE, CH>,
-                                                 hipFuncAttributeMaxDynamicSharedMemorySize, (int)shm_max);
-        if (e != hipSuccess) return e;
-        raised.fetch_or(bit, std::memory_order_acq_rel);
-    }
+    if (const hipError_t e = raise_lds((const void*)k_qsa_select<IN_DT, KR, MODE, CH>, shm_max, raised); e != hipSuccess) return e;
     hipLaunchKernelGGL((k_qsa_select<IN_DT, KR, MODE, CH>), grid, dim3(kQsaThreads), shm, s, a);
     return hipGetLastError();
 }
@@ -984,6 +1131,42 @@ hipError_t launch_qsa_select(const QsaSelectArgs& a, int in_dtype, hipStream_t s
     const dim3 grid((nmax + kQsaChunk - 1) / kQsaChunk > 0 ? (nmax + kQsaChunk - 1) / kQsaChunk : 1, a.n);
     const int kr = select_kr(nmax);
     return in_dtype == 0 ? launch_select_dt<0>(a, kr, shm, grid, s) : launch_select_dt<1>(a, kr, shm, grid, s);
+}
+
+// The many-token form: a's tokens scored on the matrix cores, then selected (no append, no histograms).
+template <int IN_DT, int ID>
+static hipError_t launch_score(const QsaSelectArgs& a, hipStream_t s) {
+    constexpr size_t shm = (size_t)qsa_score_heads(ID) * kQsaTok * (ID + 4) * 4;
+    static std::atomic<uint64_t> raised{0};
+    if (const hipError_t e = raise_lds((const void*)k_qsa_score<IN_DT, ID>, shm, raised); e != hipSuccess) return e;
+    const dim3 grid((a.stride + kQsaScoreBlocks - 1) / kQsaScoreBlocks, (a.n + kQsaTok - 1) / kQsaTok);
+    hipLaunchKernelGGL((k_qsa_score<IN_DT, ID>), grid, dim3(256), shm, s, a);
+    return hipGetLastError();
+}
+template <int KR>
+static hipError_t launch_pick(const QsaSelectArgs& a, hipStream_t s) {
+    const size_t shm = qsa_select_lds(1, 64);
+    static std::atomic<uint64_t> raised{0};
+    if (const hipError_t e = raise_lds((const void*)k_qsa_pick<KR>, shm, raised); e != hipSuccess) return e;
+    hipLaunchKernelGGL(k_qsa_pick<KR>, dim3(a.n), dim3(kQsaThreads), shm, s, a);
+    return hipGetLastError();
+}
+
+hipError_t launch_qsa_select_many(const QsaSelectArgs& a, int in_dtype, hipStream_t s) {
+    const int kr = select_kr((a.pos + a.n) / a.CR);
+    if (kr == 0 || kr > 32 || a.stride % 4 || a.raw) return hipErrorInvalidValue;
+    auto score = [&](auto dt) {
+        constexpr int DT = decltype(dt)::value;
+        switch (a.ID) {
+            case 64: return launch_score<DT, 64>(a, s);
+            case 128: return launch_score<DT, 128>(a, s);
+            case 192: return launch_score<DT, 192>(a, s);
+            default: return launch_score<DT, 256>(a, s);
+        }
+    };
+    const hipError_t e = in_dtype == 0 ? score(std::integral_constant<int, 0>{}) : score(std::integral_constant<int, 1>{});
+    if (e != hipSuccess) return e;
+    return kr == 8 ? launch_pick<8>(a, s) : kr == 16 ? launch_pick<16>(a, s) : launch_pick<32>(a, s);
 }
 
 hipError_t launch_qsa_key_bits(const QsaKeyBitsArgs& a, hipStream_t s) {

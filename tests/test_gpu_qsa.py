@@ -102,6 +102,28 @@ CASES = {
 TIE_PERIOD = {"ties_cr8": 37, "ties_cr4_8k": 37, "ties_cr2_64k": 101, "ties_long_cr2": 1009}  # blocks
 
 
+# Calls that score on the matrix cores (16 tokens and more, 896 workgroups of 64 blocks): every indexer width, heads
+# in one and several groups, dense tokens beside selecting ones, partial token groups, 8, 16 and 32 keys a selecting
+# thread, exact ties
+MANY = {
+    "many_dense_first": (QsaShape(2, 64, 2, 3200, 64), 4096, [(0, 3000, 0), (3000, 300, 1)], "f32"),
+    "many_heads9_64": (QsaShape(9, 64, 4, 512, 32), 4096, [(0, 3000, 0), (3000, 80, 1)], "f32"),
+    "many_heads5_128": (QsaShape(5, 128, 4, 256, 64), 6000, [(0, 5000, 0), (5000, 50, 1)], "bf16"),
+    "many_heads3_192": (QsaShape(3, 192, 3, 48, 64), 4096, [(0, 4000, 0), (4000, 50, 1)], "f32"),
+    "many_heads3_256": (QsaShape(3, 256, 2, 100, 128), 4096, [(0, 3000, 0), (3000, 40, 1)], "f32"),
+    "many_16_keys": (QsaShape(1, 64, 2, 128, 64), 20100, [(0, 20000, 0), (20000, 17, 1)], "f32"),
+    "many_32_keys": (QsaShape(1, 64, 2, 128, 0), 40100, [(0, 40000, 0), (40000, 31, 1)], "bf16"),
+    "ties_many": (QsaShape(2, 128, 8, 8 * 100, 64), 8200, [(0, 8000, 0), (8000, 60, 1)], "f32"),
+    "zeros_many": (QsaShape(2, 128, 4, 256, 64), 8200, [(0, 8000, 0), (8000, 33, 1)], "f32"),
+}
+TIE_PERIOD["ties_many"] = 37
+
+
+@pytest.mark.parametrize("name", list(MANY))
+def test_qsa_many_tokens_match_oracle(qw, oracle, name):
+    _indexer_case(qw, oracle, name, *MANY[name])
+
+
 @pytest.mark.parametrize("name", list(CASES))
 def test_qsa_indexer_matches_oracle(qw, oracle, name):
     _indexer_case(qw, oracle, name, *CASES[name])
