@@ -10,6 +10,7 @@ tests/conftest.py, bench.py and __graft_entry__.py) under the module name `qwatt
 """
 import ctypes
 import os
+import struct
 
 import torch  # loads the HIP runtime that libqwattn.so then shares
 
@@ -40,6 +41,10 @@ class MatOut(ctypes.Structure):
     """qwattn_mat_out: one matrix of qwattn_mat_multi and its output."""
     _fields_ = [("w", ctypes.c_void_p), ("s", ctypes.c_void_p), ("rows", ctypes.c_int), ("y", ctypes.c_void_p),
                 ("y_stride", ctypes.c_int), ("post", ctypes.c_int), ("post_scale", ctypes.c_float)]
+
+
+_MAT_OUT = struct.Struct("@PPI4xPIif4x")  # MatOut's layout; packing it costs a quarter of a ctypes.Structure
+assert _MAT_OUT.size == ctypes.sizeof(MatOut)
 
 
 _lib = None
@@ -123,44 +128,59 @@ def header_functions():
     return sorted(set(re.findall(r"^\s*(?:int|const char\*)\s+(qwattn_\w+)\s*\(", text, re.M)))
 
 
+# A decode layer's launches take 25 us on the card, and its three calls took 36 us to issue through ctypes objects,
+# torch.cuda.Stream objects and repeated tensor attributes: addresses and streams go to ctypes as plain integers,
+# and each tensor attribute is read once. Layers of one token at 4,096 keys: 36.9 -> 24.3 us each.
 def _ptr(t):
-    return None if t is None else ctypes.c_void_p(t.data_ptr())
+    return None if t is None else t.data_ptr()
+
+
+_raw_stream = torch._C._cuda_getCurrentRawStream
+_cuda_device = torch._C._cuda_getDevice
 
 
 def _stream(stream):
-    s = stream if stream is not None else torch.cuda.current_stream()
-    return ctypes.c_void_p(s.cuda_stream)
+    """The handle of `stream`, or of the current device's current stream."""
+    if stream is not None:
+        return stream.cuda_stream
+    if torch.cuda.is_initialized():
+        return _raw_stream(_cuda_device())
+    return torch.cuda.current_stream().cuda_stream
 
 
+_F32, _I8 = torch.float32, torch.int8
 _DT = {torch.float32: F32, torch.bfloat16: BF16, torch.float16: F16}
 
 
 def _check_weights(w, s):
     """(rows, cols) of a projection's weights: int8 [rows, cols] with float32 scales s [rows, cols/32] (planar
     Q8_0), or float32 [rows, cols] with s None; both contiguous, as the C ABI reads them."""
-    if w.dim() != 2 or not w.is_contiguous():
-        raise ValueError(f"weights must be a contiguous [rows, cols] matrix, got shape {tuple(w.shape)}")
-    rows, cols = w.shape
+    shape = w.shape
+    if len(shape) != 2 or not w.is_contiguous():
+        raise ValueError(f"weights must be a contiguous [rows, cols] matrix, got shape {tuple(shape)}")
+    rows, cols = shape
     if s is None:
-        if w.dtype != torch.float32:
+        if w.dtype != _F32:
             raise ValueError(f"float weights must be float32, got {w.dtype} (int8 weights need scales)")
     else:
-        if w.dtype != torch.int8:
+        if w.dtype != _I8:
             raise ValueError(f"Q8 weights must be int8, got {w.dtype}")
-        if s.dtype != torch.float32 or not s.is_contiguous() or tuple(s.shape) != (rows, cols // 32):
+        if s.dtype != _F32 or not s.is_contiguous() or s.shape != (rows, cols // 32):
             raise ValueError(f"Q8 scales must be contiguous float32 [{rows}, {cols // 32}], got {s.dtype} "
                              f"{tuple(s.shape)}")
     return rows, cols
 
 
 def _check_rows(t, name, width, n=None):
-    """A float32 [n, >= width] operand with unit column stride (row stride free)."""
-    if t.dtype != torch.float32 or t.dim() != 2 or t.stride(1) != 1:
+    """A float32 [n, >= width] operand with unit column stride (row stride free); returns (rows, row stride)."""
+    shape, stride = t.shape, t.stride()
+    if t.dtype != _F32 or len(shape) != 2 or stride[1] != 1:
         raise ValueError(f"{name} must be float32 [n, >= {width}] with unit column stride")
-    if t.shape[1] < width:
-        raise ValueError(f"{name} has {t.shape[1]} columns, needs >= {width}")
-    if n is not None and t.shape[0] < n:
-        raise ValueError(f"{name} has {t.shape[0]} rows, needs >= {n}")
+    if shape[1] < width:
+        raise ValueError(f"{name} has {shape[1]} columns, needs >= {width}")
+    if n is not None and shape[0] < n:
+        raise ValueError(f"{name} has {shape[0]} rows, needs >= {n}")
+    return shape[0], stride[0]
 
 
 BLK = 32  # positions per cache block
@@ -319,30 +339,33 @@ class Attention:
         """y [n, >= rows] = x [n, >= cols] W^T (Qwen4Vulkan::mat): W planar Q8 (w int8 [rows, cols] with s
         [rows, cols/32]) or float32 w [rows, cols]; post 1 applies silu(y * post_scale)."""
         rows, cols = _check_weights(w, s)
-        _check_rows(x, "x", cols)
-        _check_rows(y, "y", rows, n=x.shape[0])
-        self._check(self.lib.qwattn_mat(self.h, _stream(stream), _ptr(w), _ptr(s), int(s is not None), rows, cols,
-                                        _ptr(x), x.stride(0), _ptr(y), y.stride(0), x.shape[0], post, post_scale))
+        n, x_stride = _check_rows(x, "x", cols)
+        y_stride = _check_rows(y, "y", rows, n)[1]
+        self._check(self.lib.qwattn_mat(self.h, _stream(stream), w.data_ptr(), _ptr(s), int(s is not None), rows, cols,
+                                        x.data_ptr(), x_stride, y.data_ptr(), y_stride, n, post, post_scale))
 
     def mat_multi(self, x, outs, stream=None):
         """Several projections of x in one call (qwattn_mat_multi): outs = [(y, w, s), ...] (s None for float32
         weights, all of one kind and one column count), each as in mat."""
         if not outs:
             raise ValueError("mat_multi: no matrices")
-        q8 = outs[0][2] is not None
-        cols = _check_weights(outs[0][1], outs[0][2])[1]
-        _check_rows(x, "x", cols)
-        arr = (MatOut * len(outs))()
+        _, w, s = outs[0]
+        q8 = s is not None
+        first = _check_weights(w, s)
+        cols = first[1]
+        n, x_stride = _check_rows(x, "x", cols)
+        mats = bytearray()
         for i, (y, w, s) in enumerate(outs):
             if (s is not None) != q8:
                 raise ValueError(f"mat_multi: matrix {i} mixes Q8 and float32 weights")
-            rows, c = _check_weights(w, s)
+            rows, c = _check_weights(w, s) if i else first
             if c != cols:
                 raise ValueError(f"mat_multi: matrix {i} has {c} columns, matrix 0 has {cols}")
-            _check_rows(y, f"y[{i}]", rows, n=x.shape[0])
-            arr[i] = MatOut(_ptr(w), _ptr(s), rows, _ptr(y), y.stride(0), 0, 0.0)
-        self._check(self.lib.qwattn_mat_multi(self.h, _stream(stream), ctypes.cast(arr, ctypes.c_void_p), len(outs),
-                                              int(q8), cols, _ptr(x), x.stride(0), x.shape[0]))
+            y_stride = _check_rows(y, f"y[{i}]", rows, n)[1]
+            mats += _MAT_OUT.pack(w.data_ptr(), s.data_ptr() if q8 else 0, rows & 0xFFFFFFFF, y.data_ptr(),
+                                  y_stride & 0xFFFFFFFF, 0, 0.0)  # 32 bits as ctypes.c_int takes them
+        self._check(self.lib.qwattn_mat_multi(self.h, _stream(stream), bytes(mats), len(outs), int(q8), cols,
+                                              x.data_ptr(), x_stride, n))
 
     def qsa_key_bits(self, mask, cr, pos, n, key_bits, stream=None):
         """Per-key visibility bits [n, kb_words] from a block mask [n, mask_words] (shaders/attention.comp:35-43)."""
