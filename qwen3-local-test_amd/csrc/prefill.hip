@@ -539,13 +539,14 @@ __device__ __forceinline__ void pf_segment(const PrefillArgs& a, int kvh, int qt
     int kp = 0, kt = tile(lo), k1 = tile(lo + 1), k2 = tile(lo + 2);
     auto iter = [&](auto do_pv, int en) __attribute__((always_inline)) {
         constexpr bool DO_PV = decltype(do_pv)::value;
+        if constexpr (!QSA) kt = en, k2 = en + 2;
 #pragma unroll
         for (int cq = 0; cq < 4; cq++) sc[cq] = sn[cq];
         // this wave's copies are complete; after the barrier every wave's are, and every wave is done
         // with the buffers this iteration's copies overwrite (K tile kt, V tile kt-2)
         __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0)
         __syncthreads();
-        const int k3 = QSA ? tile(en + 3) : en + 3;
+        const int k3 = QSA ? tile(en + 3) : 0;
         if (DO_PV && (kp + 1) * PF_KT > maxlen) {
             zero_tail(sV((en - 1) & 1), kp);
             __syncthreads();
@@ -573,7 +574,8 @@ __device__ __forceinline__ void pf_segment(const PrefillArgs& a, int kvh, int qt
         const f16* Kb = sK((en + 1) & 1) + foff_lane;  // the next tile (stale past the last: unused)
         const f16* Vb = sV((en + 1) & 1) + foff_lane;  // the tile before (no P.V on the first)
         step(do_pv, Kb, Vb, en, kt, k2);
-        kp = kt, kt = k1, k1 = k2, k2 = k3;
+        kp = kt;
+        if constexpr (QSA) kt = k1, k1 = k2, k2 = k3;
         if (any_rescale) {
 #pragma unroll
             for (int dt = 0; dt < NDT; dt++) acc[dt] *= corr;
