@@ -431,8 +431,8 @@ def run_workload(wl, steps, warmup, graph):
                   "us_qkv_projections": statistics.mean(k_first), "us_attention_and_output": statistics.mean(k_second),
                   "us_main_is": "k_decode_ld alone"})
     elif getattr(wl, "mat", False):
-        kern = ("k_gemm<q8> (tiled MFMA GEMM, one launch a projection" if wl.n >= 16 else
-                "k_mat_multi<q8> + k_mat_q8 (matrix-vector: query + gate, key and value in one launch, then output")
+        kern = ("k_gemm_q8 (tiled MFMA GEMM, a launch each for query + gate and output; k_mat_tok: key and value in one" if wl.n >= 16 else
+                ("k_mat_tok (token-tile MFMA" if wl.n > 1 else "k_mat_multi<q8> + k_mat_q8 (matrix-vector") + ": query + gate, key and value in one launch, then output")
         r.update({"kernel": kern + "; the per-launch figure is the 8,192 x 2,048 query + gate projection alone)",
                   "us_first_event": statistics.mean(k_first)})
     elif getattr(wl, "qsa", False):
