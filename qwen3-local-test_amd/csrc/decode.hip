@@ -180,16 +180,23 @@ __device__ __forceinline__ void merge_batch(float& M, float& L, f32x4& O, const 
     M = mx;
 }
 
+// The value of lane l ^ 32, for a value that is the same in the lanes of each half.
+__device__ __forceinline__ float other_half(float x) {
+    const auto b = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+    return __uint_as_float((threadIdx.x & 32) ? b[0] : b[1]);
+}
+
 // In-launch log-sum-exp combine of the one-launch decode (attn_combine.comp:13-29): one workgroup per
 // (output row (t, h), slice of DW = D / nds dims), one of the last chunks of its KV head or 16-row slice
 // once its own partials are out, merges that row's split partials over its dims as they arrive. A
 // streaming workgroup stores its rows' unnormalized o[D] (device-coherent stores), waits for them to be
 // acknowledged, then stores each row's record (m, l, 64-bit tag): a record carrying this launch's tag
-// guarantees the row's o is visible. The combiner takes the splits in windows of kCombSlots: wave w owns
-// the kCombGroup splits [wb + 32 w, wb + 32 w + 32) of window wb, lane j < 32 polling split wb + 32 w + j's
+// guarantees the row's o is visible. The combiner takes the splits in windows of four groups of GS = 32 (64
+// past 128 splits, so that the 256 of a single KV head are one window; below): wave w owns the splits
+// [wb + GS w, wb + GS w + GS) of window wb, lane j < GS polling split wb + GS w + j's
 // record (one 16-byte device-coherent load per round); each split that has arrived has its DW dims loaded
 // straight into the wave's registers, 16 bytes a lane: lane group g (LPP = DW / 4 lanes) holds splits
-// g NL .. g NL + NL - 1 of the wave's 32. Once its group is complete the wave takes the group's max and
+// g NL .. g NL + NL - 1 of the wave's. Once its group is complete the wave takes the group's max and
 // weights (wave reductions, the weights broadcast through LDS), its weighted sum per lane and then across
 // the lane groups; the window's four group results meet in LDS and merge into the running (M, L, O) in
 // group order — a fixed order, so the result does not depend on which split arrives first. Splits with
@@ -198,11 +205,11 @@ __device__ __forceinline__ void merge_batch(float& M, float& L, f32x4& O, const 
 // kEpochStep. Every wait is bounded (a.spin_max polling rounds); a combiner that gives up reports
 // kWaitCombineFlags and merges whatever its registers hold. The host keeps the combiners at half of each
 // KV head's (slice's) chunks or fewer, so every wait ends while more CUs than that are free to the launch.
-template <int D, int IN_DT, int DW>
+template <int D, int IN_DT, int DW, int GS>
 __device__ __forceinline__ void combine_slice(const DecodeArgs& a, unsigned char* smem, int r, int ds) {
-    constexpr int NS = kCombSlots, GS = kCombGroup;
+    constexpr int NS = 4 * GS;
     constexpr int LPP = DW / 4, PPL = 64 / LPP, NL = GS / PPL;  // lanes a split, splits a load, loads a wave
-    static_assert(NS == 4 * GS && GS == 32, "one group of 32 splits per wave and window");
+    static_assert(GS == 32 || GS == 64, "a lane a split of the wave's group");
     static_assert(DW % 16 == 0 && DW <= 256 && DW <= D, "16 to 256 dims a combiner, 4 a lane");
     float* s_go = reinterpret_cast<float*>(smem);  // [4][DW] the window's group sums
     float* s_gm = s_go + 4 * DW;                    // [4] group maxima (log2 units)
@@ -252,10 +259,12 @@ __device__ __forceinline__ void combine_slice(const DecodeArgs& a, unsigned char
         // the group's max and weights: lane j < nz holds split z0 + j's (m, l)
         // (DPP/permlane butterflies over the 32 lanes: no LDS round trips)
         const bool use = lane < nz && lj > 0.f;
-        const float mg = max32(use ? mj : kNegInf);
+        float mg = max32(use ? mj : kNegInf);
+        if constexpr (GS == 64) mg = fmaxf(mg, other_half(mg));
         const float w = use ? exp2_fast(mj - mg) : 0.f;
-        const float lsum = sum32(lj * w);
-        // the weights to every lane through LDS (broadcast reads): lane j < 32 holds split z0 + j's
+        float lsum = sum32(lj * w);
+        if constexpr (GS == 64) lsum += other_half(lsum);
+        // the weights to every lane through LDS (broadcast reads): lane j < GS holds split z0 + j's
         if (lane < GS) s_w[wave * GS + lane] = w;
         float wv[NL];
 #pragma unroll
@@ -306,14 +315,20 @@ __device__ __forceinline__ void combine_slice(const DecodeArgs& a, unsigned char
     }
 }
 
-// The combiner of output row r, dims slice ds of a.nds (1, 2, 4 or 8: host-checked)
-template <int D, int IN_DT>
+// The combiner of output row r, dims slice ds of a.nds (1, 2, 4 or 8: host-checked). WIDE (k_decode_ld): past
+// kCombSlots splits a wave polls 64 at once, so that a single KV head's 256 parts take one window instead of two in
+// turn: 2 query heads on one KV head, D = 256, at 4K / 32K / 256K 11.5 / 16.1 / 52.4 -> 10.8 / 14.8 / 51.3 us; 4 on
+// one, D = 64, 8.9 / 10.9 / 19.4 -> 7.8 / 9.3 / 18.4. Not in k_decode, whose tile loop has no registers to spare
+// for it (the 4-token verify layer at 32K 42.7 -> 44.4 us with it).
+template <int D, int IN_DT, bool WIDE>
 __device__ __forceinline__ void combine_row(const DecodeArgs& a, unsigned char* smem, int r, int ds) {
     if constexpr (D / 8 >= 16)
-        if (a.nds == 8) return combine_slice<D, IN_DT, D / 8>(a, smem, r, ds);
-    if (a.nds == 4) combine_slice<D, IN_DT, D / 4>(a, smem, r, ds);
-    else if (a.nds == 2) combine_slice<D, IN_DT, D / 2>(a, smem, r, ds);
-    else combine_slice<D, IN_DT, D>(a, smem, r, ds);
+        if (a.nds == 8) return combine_slice<D, IN_DT, D / 8, kCombGroup>(a, smem, r, ds);
+    if constexpr (WIDE)
+        if (a.nds == 4 && a.n_split > kCombSlots) return combine_slice<D, IN_DT, D / 4, 2 * kCombGroup>(a, smem, r, ds);
+    if (a.nds == 4) combine_slice<D, IN_DT, D / 4, kCombGroup>(a, smem, r, ds);
+    else if (a.nds == 2) combine_slice<D, IN_DT, D / 2, kCombGroup>(a, smem, r, ds);
+    else combine_slice<D, IN_DT, D, kCombGroup>(a, smem, r, ds);
 }
 
 template <int D, int FUSED, int IN_DT, int QSA>
@@ -716,7 +731,7 @@ __global__ __launch_bounds__(256, 1) void k_decode(DecodeArgs a) {
             const int zc = z - (a.n_split - rows * a.nds);
             if (zc >= 0) {
                 const int rl = r0 + zc % rows, t = rl / G, h = kvh * G + rl % G;
-                combine_row<D, IN_DT>(a, s_u, t * a.NH + h, zc / rows);
+                combine_row<D, IN_DT, false>(a, s_u, t * a.NH + h, zc / rows);
             }
         }
     }
@@ -1214,7 +1229,7 @@ __global__ __launch_bounds__(256, 1) void k_decode_ld(DecodeArgs a) {
             if (zc >= 0) {
                 __syncthreads();
                 const int rl = zc % rows;
-                combine_row<D, IN_DT>(a, smem, (rl / G) * a.NH + kvh * G + rl % G, zc / rows);
+                combine_row<D, IN_DT, true>(a, smem, (rl / G) * a.NH + kvh * G + rl % G, zc / rows);
             }
         }
     }
@@ -1224,7 +1239,7 @@ template <int D, int QSA>
 constexpr size_t decode_ld_lds() {
     // ring + Q fragments (+ QSA: the visible-tile list and its key words)
     const size_t stream = (size_t)2 * 2 * 2 * kBlk * D * 2 + (size_t)(D / 32) * 64 * 8 * 2 + (QSA ? kQsaTiles * 9 * 4 : 0);
-    const size_t comb = (size_t)4 * (D + 2 + kCombGroup) * 4;  // combiner: a window's group sums, maxima, sums, weights
+    const size_t comb = (size_t)4 * (D + 2 + 2 * kCombGroup) * 4;  // combiner: a window's group sums, maxima, sums, weights
     return stream > comb ? stream : comb;
 }
 

@@ -86,8 +86,8 @@ hipError_t launch_decode(const DecodeArgs& a, int D, bool fused, int in_dtype, h
 // less, and floor(counter / K) + 1 is the epoch of the next launch — also for a participant that reads the
 // counter after some combiners of its own launch are done.
 constexpr unsigned kEpochStep = 840;
-constexpr int kCombSlots = 128;       // split partials a combining workgroup stages in LDS at once
-constexpr int kCombGroup = 32;        // splits merged together (in a fixed order) once all are staged
+constexpr int kCombGroup = 32;        // splits a combining wave merges together (twice as many past kCombSlots)
+constexpr int kCombSlots = 4 * kCombGroup;  // splits the four waves take at once
 
 struct CombineArgs {
     const float* part_o;

@@ -166,11 +166,14 @@ bool tail_launch(const qwattn_config& g, int n, int S) {
 
 // Dim slices per output row of that combine: the most of 4, 2, 1 that keeps the combiners at half of a
 // head's (slice's) chunks or fewer (4 at decode: 32 of 128 chunks; 2 at the 4-token verify: 32 of 64);
-// each combiner then loads and sums D / slices dims of every split.
+// each combiner then loads and sums D / slices dims of every split. Two at most for 9 rows and more: 64
+// combiners polling a slice's 128 chunks cost more than their shorter sums save (16 query heads on 2 KV
+// heads, D = 256, two tokens at 4K / 16K / 32K 16.7 / 20.6 / 27.0 us with four, 15.9 / 19.9 / 26.4 with two;
+// 8 on 2, D = 128, four tokens 11.3 / 12.2 / 14.7 and 10.6 / 11.6 / 14.0).
 int combine_slices(const qwattn_config& g, int n, int S) {
     const int rows = std::min(n * (g.n_heads / g.n_kv_heads), 16);
     for (int k : {4, 2})
-        if (k > 0 && 2 * rows * k <= S && g.head_dim / k >= 16) return k;
+        if ((k <= 2 || rows <= 8) && 2 * rows * k <= S && g.head_dim / k >= 16) return k;
     return 1;
 }
 

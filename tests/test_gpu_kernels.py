@@ -344,6 +344,17 @@ def test_decode_one_launch_parity(qw, oracle, s, pos, n, n_split, dtype):
     assert_parity(host(out), ref, f"{s} pos={pos} n={n} splits={used}")
 
 
+# the combine's window of 256 splits (64 a wave) from 129 on: its edges, a partly filled second window, one KV
+# head of 8 rows or fewer (four dim slices) and of 9 to 16 (two)
+COMBINE_WINDOWS = [(TINY, 8400, 1, 129), (TINY, 8400, 1, 256), (TINY_GGUF, 8400, 1, 192), (TINY_GGUF, 8170, 2, 0),
+                   (TINY, 8400, 4, 129), (TINY, 8191, 4, 0), (TINY_GGUF, 8400, 8, 200), (TINY_GGUF, 8800, 8, 262)]
+
+
+@pytest.mark.parametrize("s,pos,n,n_split", COMBINE_WINDOWS, ids=lambda v: repr(v))
+def test_decode_combine_windows(qw, oracle, s, pos, n, n_split):
+    test_decode_one_launch_parity(qw, oracle, s, pos, n, n_split, "f32")
+
+
 def test_decode_one_launch_equals_two_launches(qw):
     """The in-launch combine merges what qwattn_combine merges: over a run of calls on one context with
     changing token counts (decode n=1 on the loader-wave kernel, verify n=4 on two 16-row slices, combined
