@@ -107,7 +107,8 @@ struct PrefillArgs {
     int pos, n, NH, NKV;
     float q_scale;
     int cap;              // capacity (positions) of the caches kc, vc
-    float* part;          // [NKV][slots][parts][kPfWaves][pf_part_floats(D)]: partials of split query tiles
+    float* part;          // [NKV * slots regions of pf_region][kPfWaves][pf_part_floats(D)]: partials of split query
+                          // tiles
     int* cnt;             // [NKV][slots][kPfWaves] arrival counters, zero between launches
     int slots;            // split tiles per KV head: pf_split_slots(n_qt, split_all)
     int split_all;        // 0: short and long tiles paired (two parts a long tile); else the parts, a workgroup
@@ -139,6 +140,34 @@ inline int pf_parts(int n_qt, int nkv, int n_cu, int nt) {
     int p = 2;
     while (p < 16 && 2 * p * n_qt * nkv <= n_cu && nt >= 48 && 4 * p * p <= nt) p *= 2;
     return p;
+}
+// The key tiles [lo, hi) of part `part` of a query tile that has nt of them, split_all parts asked for (a power of
+// two): equal runs, a tile to a part where there are fewer tiles than parts (`parts` of them, the rest empty).
+struct PfPart {
+    int parts, lo, hi;
+};
+__host__ __device__ constexpr PfPart pf_part(int nt, int split_all, int part) {
+    if (nt < split_all) return PfPart{nt, part, part + 1};
+    const int lg = __builtin_ctz((unsigned)split_all);
+    return PfPart{split_all, nt * part >> lg, nt * (part + 1) >> lg};
+}
+// The partials' region of part `part` of split slot `slot` (counted over the KV heads). The stride is the launch's
+// part count, never a tile's own: tiles with fewer parts than others would share regions with their neighbours.
+__host__ __device__ constexpr int pf_region(int slot, int part, int split_all) {
+    return slot * (split_all ? split_all : 2) + part;
+}
+// Split slots and partial regions per KV head that launches of up to qt_max query tiles need on n_cu CUs: a pair of
+// query tiles each (paired schedule: two regions) or a tile each (split schedule: pf_parts regions), at least one
+// slot.
+constexpr int pf_slots_per_head(int qt_max, int nkv, int n_cu) {
+    const int split = qt_max < n_cu / (2 * nkv) ? qt_max : n_cu / (2 * nkv);
+    const int m = qt_max / 2 > split ? qt_max / 2 : split;
+    return m > 1 ? m : 1;
+}
+constexpr int pf_regions_per_head(int qt_max, int nkv, int n_cu) {
+    const int split = 16 * qt_max < n_cu / nkv ? 16 * qt_max : n_cu / nkv;
+    const int m = qt_max > split ? qt_max : split;
+    return m > 2 ? m : 2;
 }
 // Waves of a prefill workgroup (16 query rows each).
 constexpr int kPfWaves = 8;

@@ -641,7 +641,7 @@ __device__ __forceinline__ void pf_segment(const PrefillArgs& a, int kvh, int qt
         // the tile has its own region
         constexpr int PSTR = pf_part_floats(D);
         auto region = [&](int part) {
-            return __builtin_amdgcn_make_buffer_rsrc(a.part + (((size_t)slot * parts + part) * kPfWaves + wave) * PSTR,
+            return __builtin_amdgcn_make_buffer_rsrc(a.part + ((size_t)pf_region(slot, part, SPLIT ? a.split_all : 0) * kPfWaves + wave) * PSTR,
                                                      (short)0, PSTR * 4, 0x00020000);
         };
         int* cw = a.cnt + slot * kPfWaves + wave;
@@ -806,11 +806,9 @@ __global__ __launch_bounds__(64 * kPfWaves, 1) void k_prefill(PrefillArgs a) {
         const int lg = __builtin_ctz((unsigned)a.split_all);
         const int qt = n_qt - 1 - (j >> lg), part = a.split_all - 1 - (j & (a.split_all - 1));
         const int nt = tiles(qt, list0);
-        parts0 = min(a.split_all, nt);  // a part holds a tile at least
-        if (part >= parts0) return;
-        q0 = qt, own0 = part;
-        lo0 = nt < a.split_all ? part : nt * part >> lg;
-        hi0 = nt < a.split_all ? part + 1 : nt * (part + 1) >> lg;
+        const PfPart pt = pf_part(nt, a.split_all, part);
+        if (part >= pt.parts) return;
+        q0 = qt, own0 = part, parts0 = pt.parts, lo0 = pt.lo, hi0 = pt.hi;
         slot0 = parts0 > 1 ? kvh * a.slots + qt : -1;
     } else if (j >= 2 * np) {  // the middle tile
         q0 = np, lo0 = 0, hi0 = tiles(np, list0), slot0 = -1;

@@ -256,13 +256,10 @@ int qwattn_create(qwattn_ctx** out, int device, const qwattn_config* cfg) {
         return fail(nullptr, QWATTN_EINVAL, "max_splits %d: the split partials would exceed 2 GiB", cfg->max_splits);
     }
     const size_t qn = (size_t)cfg->max_tokens * NH * D;
-    // prefill split slots per KV head: a pair of query tiles each (paired schedule) or a tile each (split
-    // schedule, only while two workgroups per tile fit the CUs), at least one so the pointers are never
-    // null; kPfWaves waves each, a partial region per part of a split tile (two of a pair's long tile, up to 16
-    // while the parts' workgroups fit the CUs)
+    // prefill split slots and partial regions per KV head, kPfWaves waves each
     const int qt_max = qw::pf_query_tiles(cfg->max_tokens, NH / NKV);
-    c->pf_slots_per_head = std::max(1, std::max(qt_max / 2, std::min(qt_max, c->n_cu / (2 * NKV))));
-    c->pf_parts_per_head = std::max(2, std::max(qt_max, std::min(16 * qt_max, c->n_cu / NKV)));
+    c->pf_slots_per_head = qw::pf_slots_per_head(qt_max, NKV, c->n_cu);
+    c->pf_parts_per_head = qw::pf_regions_per_head(qt_max, NKV, c->n_cu);
     const size_t pf_slots = (size_t)NKV * c->pf_slots_per_head * qw::kPfWaves;
     const size_t pf_parts = (size_t)NKV * c->pf_parts_per_head * qw::kPfWaves;
     c->qsa_hist_n = std::min(cfg->max_tokens, qw::kQsaHistTokens);
@@ -670,7 +667,9 @@ static int prefill_args(qwattn_ctx* c, const void* q, const void* kcache, const 
     *a = qw::PrefillArgs{q, (const uint16_t*)kcache, (const uint16_t*)vcache, qg, out, pos, n, g.n_heads,
                          g.n_kv_heads, qw::kLog2eHost / std::sqrt((float)g.head_dim), kv_cap, c->pf_part, c->pf_cnt,
                          qw::pf_split_slots(n_qt, split_all), split_all, nullptr, nullptr, 0, g.rms_eps, nullptr, 0, 0};
-    if (a->slots > c->pf_slots_per_head || a->slots * std::max(2, split_all) > c->pf_parts_per_head) return fail(c, QWATTN_EINVAL, "prefill: %d split slots > %d", a->slots, c->pf_slots_per_head);
+    if (a->slots > c->pf_slots_per_head || qw::pf_region(a->slots, 0, split_all) > c->pf_parts_per_head)
+        return fail(c, QWATTN_EINVAL, "prefill: %d split slots of %d parts, the context holds %d slots and %d parts", a->slots,
+                    std::max(2, split_all), c->pf_slots_per_head, c->pf_parts_per_head);
     return QWATTN_OK;
 }
 

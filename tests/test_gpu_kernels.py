@@ -548,11 +548,15 @@ def test_prefill_parity(qw, oracle, s, pos, n):
     assert_rows_parity(out, ref, f"{s} pos={pos} n={n}")
 
 
-# Small chunks on long contexts: every tile's keys over 4, 8 and 16 workgroups, and over fewer than asked for where
-# a tile has fewer key tiles
-@pytest.mark.parametrize("s,pos,n", [(QWEN3_NEXT, 1500, 300), (QWEN3_NEXT, 4060, 40), (QWEN3_NEXT, 16411, 37),
-                                     (TINY, 17000, 33), (D128, 5000, 70)], ids=lambda v: repr(v))
-def test_prefill_many_parts(qw, oracle, s, pos, n):
+# Small chunks on long contexts: every tile's keys over 2, 4, 8 and 16 workgroups; and a prompt of one head a KV head
+# from position 0, whose first tiles have fewer key tiles (2) than there are parts (4)
+@pytest.mark.parametrize("s,pos,n,parts", [
+    (QWEN3_NEXT, 1500, 300, {2}), (QWEN3_NEXT, 3000, 200, {4}), (QWEN3_NEXT, 4060, 40, {8}), (QWEN3_NEXT, 16411, 37, {16}),
+    (TINY, 17000, 33, {16}), (D128, 5000, 70, {8}), (Shape(2, 2, 256, 64), 0, 3072, {2, 4})], ids=lambda v: repr(v))
+def test_prefill_many_parts(qw, oracle, walk, s, pos, n, parts):
+    cus = torch.cuda.get_device_properties(0).multi_processor_count
+    got = walk([(s.NH, s.NKV, pos, n, n, [])], cus)
+    assert (got["mixed"], got["worst"]) == (int(len(parts) > 1), max(parts))
     test_prefill_parity(qw, oracle, s, pos, n)
 
 

@@ -465,6 +465,55 @@ def test_prefill_qsa_sparse_tiles(qw, oracle, pos, n, dt, cr, density):
     test_prefill_qsa_parity(qw, oracle, QWEN3_NEXT, pos, n, dt, cr, density, "prefill")
 
 
+# Query tiles (16 tokens) that see unequal numbers of 64-key tiles, below and above the launch's parts (16, 8 and 4),
+# on two KV heads, so that tiles with few parts lie between tiles with many in the partials' workspace
+@pytest.mark.parametrize("dt", ["f32", "bf16"])
+@pytest.mark.parametrize("pos,n,see,parts", [(16384, 64, [9, 10, 12, 16], 16), (16384, 96, [1, 2, 9, 10, 12, 40], 16),
+                                             (16448, 60, [30, 3, 1, 2], 16), (4096, 100, [2, 7, 3, 20, 5, 11, 1], 8),
+                                             (8000, 330, [1, 3, 2, 9, 30], 4)], ids=lambda v: str(v))
+def test_prefill_qsa_unequal_parts(qw, oracle, walk, pos, n, see, parts, dt):
+    import oracle as orc
+    s, cr = QWEN3_NEXT, 64
+    tok = 128 // s.G
+    rows, cap = pos + n, capacity(pos + n)
+    r = np.random.default_rng(pos + n)
+    bits = np.zeros((n, (rows // cr // 32 + 1) * 32), bool)
+    for qt in range((n + tok - 1) // tok):  # the tile's tokens share its blocks; the tail's tile is the last they see
+        last = (pos + min(n, (qt + 1) * tok) - 1) // cr
+        first = (pos + qt * tok + 1) // cr  # tiles from the first token's tail on are seen in any case
+        took = r.choice(first, max(0, see[qt % len(see)] - (last - first + 1)), replace=False)
+        bits[qt * tok:(qt + 1) * tok, took] = True
+    mask = (bits.reshape(n, -1, 32).astype(np.uint64) << np.arange(32, dtype=np.uint64)).sum(axis=2).astype(np.uint32)
+    words = orc.qsa_key_bits(mask, pos, n, cr)
+    # what each query tile sees, and that the launch's tiles differ in parts as meant
+    pairs = np.zeros((n, (words.shape[1] + 1) // 2 * 2), np.uint32)
+    pairs[:, :words.shape[1]] = words
+    any64 = (pairs[:, 0::2] | pairs[:, 1::2]) != 0
+    seen = [int(any64[t:t + tok, :(pos + min(n, t + tok) + 63) // 64].any(axis=0).sum()) for t in range(0, n, tok)]
+    cus = torch.cuda.get_device_properties(0).multi_processor_count
+    got = walk([(s.NH, s.NKV, pos, n, n, seen)], cus)
+    print(f"qsa prefill pos={pos} n={n} {dt}: tiles seen {seen}", flush=True)
+    assert got == {"split": 1, "mixed": 1, "worst": min(parts, max(seen))} and min(seen) < parts
+    k16, v16 = cache_rows(90 + pos, pos, s)
+    qg, k, v, qn, kn = projections(91 + n, n, s)
+    tdt = torch.bfloat16 if dt == "bf16" else torch.float32
+    qg_d, k_d, v_d = dev(qg).to(tdt), dev(k).to(tdt), dev(v).to(tdt)
+    ctx = make_ctx(qw, s, max_ctx=cap, max_tokens=n)
+    kc, vc = gpu_caches(qw, k16, v16, cap)
+    kbits = dev(words.view(np.int32))
+    outs = [torch.full((n, s.NH, s.D), float("nan"), device=DEV) for _ in range(3)]
+    for out in outs:
+        ctx.prefill_qsa(qg_d, k_d, v_d, dev(qn), dev(kn), ctx.rope_table(), kc, vc, cap, out, pos, n, kbits)
+    ctx.sync_status()
+    assert torch.equal(outs[0], outs[1]) and torch.equal(outs[0], outs[2])
+    rq, _, _ = oracle.qk_norm_rope(host(qg_d), host(k_d), host(v_d), 1 + qn, 1 + kn, pos, s.R, s.theta, s.eps)
+    kcache = host(qw.k_rows(kc, cap, s.NKV, s.D)[:rows])
+    vcache = host(qw.v_rows(vc, cap, s.NKV, s.D)[:rows])
+    ref = oracle.attention_qsa(rq, kcache, vcache, pos, mask, cr, host(qg_d))
+    assert_rows_parity(host(outs[0]), ref, f"qsa prefill, unequal parts, pos={pos} n={n}")
+    ctx.close()
+
+
 def test_prefill_qsa_past_list_limit(qw):
     """More key tiles than a list of visible ones holds (over 262,144 keys): every tile is read, and a few visible
     keys at both ends decide the output (float64 attention over them alone; fp16 weights: 2^-11 of each)."""
