@@ -258,4 +258,20 @@ struct MatMultiArgs {
 };
 hipError_t launch_mat_multi(const MatMultiArgs& a, bool q8, hipStream_t s);
 
+// Byte offsets of the Q8 kernels' range-checked loads; an offset of kFar or more lies outside every resource.
+constexpr unsigned kFar = 0x60000000u;
+// The Q8 GEMM's, within a tile's rows (tokens) at step k of 64 columns, two Q8 blocks of nkb: 16 weights at chunk q
+// of 4, four token values at piece q of 16, the scale of block j of 2. A last half step's second block is far.
+__host__ __device__ constexpr unsigned gemm_w_off(int row, int q, int k, int cols, int nkb) {
+    return (unsigned)(row * cols) + (2 * k + (q >> 1) < nkb ? (unsigned)(64 * k + 16 * q) : kFar);
+}
+__host__ __device__ constexpr unsigned gemm_x_off(int tok, int q, int k, int x_stride, int nkb) {
+    return (unsigned)(tok * x_stride) * 4u + (2 * k + (q >> 3) < nkb ? (unsigned)(256 * k + 16 * q) : kFar);
+}
+__host__ __device__ constexpr unsigned gemm_s_off(int row, int j, int k, int nkb) {
+    return (unsigned)(row * nkb) * 4u + (2 * k + j < nkb ? (unsigned)(8 * k + 4 * j) : kFar);
+}
+// Whether they stay below kFar, and below 2^32 with it added, over a tile's 256 rows and 128 tokens.
+constexpr bool gemm_offsets_fit(int cols, int x_stride) { return cols <= 1 << 22 && (127ll * x_stride + cols) * 4 < kFar; }
+
 }  // namespace qw

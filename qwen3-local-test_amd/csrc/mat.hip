@@ -275,7 +275,6 @@ __device__ __forceinline__ void mat_tok_body(const MatArgs& a, int bx, int by, u
     Lds& L = *reinterpret_cast<Lds*>(smem + wave * kLds);
     // rows past the matrix, tokens past the last and columns past the row (kFar added) lie outside the
     // resources: such loads read zero and cause no traffic, so no load is conditional
-    constexpr unsigned kFar = 0x60000000u;
     const int nr = min(16 * R, a.rows - r0), nt = min(16 * TT, a.n - t0);
     const __amdgpu_buffer_rsrc_t rw = __builtin_amdgcn_make_buffer_rsrc(
         const_cast<int8_t*>(static_cast<const int8_t*>(a.w)) + (size_t)r0 * a.cols, (short)0, nr * a.cols, 0x00020000);
@@ -635,7 +634,7 @@ __global__ __launch_bounds__(256, 2) void k_gemm(MatArgs a) {
 // lanes and 256 x 128 tiles, alike with 16x16x32 MFMAs in the compiler's order or pinned; 147 with 32x32x16, of
 // which the conversions take 30 and the scaling, by leaving three quarters of it out, 18.
 template <int RT, int TT, int GR, int GT>
-__global__ __launch_bounds__(512) void k_gemm_q8(MatArgs a) {
+__global__ __launch_bounds__(512, RT * TT == 1 ? 4 : 2) void k_gemm_q8(MatArgs a) {
     static_assert(GR * GT == 8, "eight waves");
     constexpr int BM = 32 * RT * GR, BN = 32 * TT * GT;
     constexpr int WL = BM / 128, XL = BN / 32;  // 16-byte loads a thread and step: weights, token rows
@@ -651,10 +650,11 @@ __global__ __launch_bounds__(512) void k_gemm_q8(MatArgs a) {
     const int r0 = (idx / TTs) * BM, t0 = (idx % TTs) * BN;
     const int nkb = a.cols >> 5, nst = (nkb + 1) >> 1;
 
-    // loads by consecutive lanes: four lanes a weight row's 64 columns, sixteen a token's, the step and the load's
-    // first row in the scalar offset. Rows and tokens past the ends, and a last half step's second block (kFar
-    // added), lie outside the resources and read zero.
-    constexpr unsigned kFar = 0x60000000u;
+    // loads by consecutive lanes: four lanes a weight row's 64 columns, sixteen a token's. Rows and tokens past the
+    // ends, and a last half step's second block, lie outside the resources and read zero: the whole offset is in the
+    // per-lane operand, since the range check leaves the scalar offset out. The additions cost nothing at 8,192 x
+    // 2,048 (2,048 tokens 152-154 us with the rows and steps in the scalar offset, 152 without) and 0.3-2 us of 92 and 55
+    // at 2,048 x 4,096 (2,048 and 1,024 tokens).
     const int wq = tid & 3, xq = tid & 15;
     const int nr = min(BM, a.rows - r0), nt = min(BN, a.n - t0);
     const __amdgpu_buffer_rsrc_t rw = __builtin_amdgcn_make_buffer_rsrc(
@@ -663,21 +663,19 @@ __global__ __launch_bounds__(512) void k_gemm_q8(MatArgs a) {
         const_cast<float*>(a.s) + (size_t)r0 * nkb, (short)0, nr * nkb * 4, 0x00020000);
     const __amdgpu_buffer_rsrc_t rx = __builtin_amdgcn_make_buffer_rsrc(
         const_cast<float*>(a.x) + (size_t)t0 * a.x_stride, (short)0, ((nt - 1) * a.x_stride + a.cols) * 4, 0x00020000);
-    const unsigned wo = (tid >> 2) * a.cols + 16 * wq, xo = ((tid >> 4) * a.x_stride + 4 * xq) * 4;
-    const unsigned so = ((tid >> 1) % BM * nkb + (tid & 1)) * 4;
     u32x4 wv[WL];
     f32x4 xv[XL];
     float sv;
     auto load_w = [&](int k) {
-        const unsigned o = 2 * k + (wq >> 1) < nkb ? wo : wo + kFar;
 #pragma unroll
         for (int i = 0; i < WL; i++)
-            wv[i] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(rw, (int)o, 128 * i * a.cols + 64 * k, 0));
-        sv = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(rs, (int)so, 8 * k, 0));
+            wv[i] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(
+                rw, (int)gemm_w_off(128 * i + (tid >> 2), wq, k, a.cols, nkb), 0, 0));
+        sv = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(rs, (int)gemm_s_off((tid >> 1) % BM, tid & 1, k, nkb), 0, 0));
     };
     auto load_x = [&](int k, int i) {
-        const unsigned o = 2 * k + (xq >> 3) < nkb ? xo : xo + kFar;
-        xv[i] = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(rx, (int)o, 128 * i * a.x_stride + 256 * k, 0));
+        xv[i] = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(
+            rx, (int)gemm_x_off(32 * i + (tid >> 4), xq, k, a.x_stride, nkb), 0, 0));
     };
     // LDS rows of 64 columns are eight 16-byte chunks, chunk q of row r at q ^ (r / 2) % 8: operand reads (16
     // rows' chunk q) and the loaders' writes are free of bank conflicts
@@ -704,10 +702,9 @@ __global__ __launch_bounds__(512) void k_gemm_q8(MatArgs a) {
             }
         }
     };
-    // the scale of a block past the row is 0: a last half step's second block adds nothing
-    auto put_s = [&](int k, unsigned char* S) {
-        if (tid < 2 * BM)
-            reinterpret_cast<float*>(S + W_B + 2 * X_B)[(tid & 1) * BM + (tid >> 1)] = 2 * k + (tid & 1) < nkb ? sv : 0.f;
+    // (the scale of a block past the row reads as 0: a last half step's second block adds nothing)
+    auto put_s = [&](unsigned char* S) {
+        if (tid < 2 * BM) reinterpret_cast<float*>(S + W_B + 2 * X_B)[(tid & 1) * BM + (tid >> 1)] = sv;
     };
 
     f32x16 acc[RT][TT];
@@ -723,7 +720,7 @@ __global__ __launch_bounds__(512) void k_gemm_q8(MatArgs a) {
     for (int i = 0; i < XL; i++) load_x(0, i);
 #pragma unroll
     for (int u = 0; u < U; u++) unit(u, smem);
-    put_s(0, smem);
+    put_s(smem);
     load_w(min(1, nst - 1));
 #pragma unroll
     for (int i = 0; i < XL; i++) load_x(min(1, nst - 1), i);
@@ -781,7 +778,7 @@ __global__ __launch_bounds__(512) void k_gemm_q8(MatArgs a) {
                 constexpr int u = u_;
                 unit(u, N);
                 if constexpr (u == UW - 1) {
-                    put_s(k + 1, N);
+                    put_s(N);
                     load_w(k2);
                 }
                 if constexpr (u >= UW && (u - UW) % 2 == 1) load_x(k2, (u - UW) / 2);
@@ -872,7 +869,7 @@ int row_groups(const MatMultiArgs& a, int r) {
 // Whether the token-tile kernel's 32-bit offsets reach every operand (up to 64 rows and tokens a workgroup).
 bool tok_fits(const MatMultiArgs& a) {
     const MatArgs& m = a.m[0];
-    return m.cols <= 1 << 24 && (63ll * m.x_stride + m.cols) * 4 < 0x60000000ll;
+    return m.cols <= 1 << 24 && (63ll * m.x_stride + m.cols) * 4 < kFar;
 }
 
 hipError_t launch_tok_any(const MatMultiArgs& a, hipStream_t s) {
@@ -935,7 +932,7 @@ const GemmTile& gemm_tile(int rows, int n) {
     return *best;
 }
 // Whether the Q8 GEMM's 32-bit offsets reach the operands.
-bool gemm_fits(const MatArgs& a) { return a.cols <= 1 << 22 && (127ll * a.x_stride + a.cols) * 4 < 0x60000000ll; }
+bool gemm_fits(const MatArgs& a) { return gemm_offsets_fit(a.cols, a.x_stride); }
 
 // Whether a Q8 matrix takes the token-tile kernel (from two tokens on): up to 64 tokens, else where its 64-row x
 // 32-token workgroups, two a CU and 0.55 us a pair and 64 columns, take less than the GEMM's tiles (8,192 x 2,048
