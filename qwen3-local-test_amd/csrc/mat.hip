@@ -223,8 +223,10 @@ __device__ __forceinline__ void split_bf16(const float (&v)[8], bf16x8& hi, bf16
 // included, takes a SIMD 2.0-2.5 ns.
 //
 // fp32 accuracy from bf16 products: an int8 weight is exact in bf16; NS = 2 splits x into hi + lo (up to 2^-18 of
-// |x| left, 2.5e-6 in an output), NS = 3 into three parts (2^-27 left: 1.1e-7, the level of fp32 sums), for the
-// token counts below 16.
+// |x| left, 2.5e-6 in an output), NS = 3 into three parts of eight bits (nothing left: 1e-7 in an output, the level of
+// fp32 sums), for the token counts below 16. bf16 ends at 2^-133, so the last part of an |x| below 2^-109 loses bits:
+// rows whose values are all that small keep 1.2e-6 at 2^-115 and 4e-5 at 2^-120 of their outputs, with two parts
+// 2.8e-6 and 4e-5.
 __device__ __forceinline__ uint32_t pk_bf16(float a, float b) {  // one v_cvt_pk_bf16_f32
     return __builtin_bit_cast(uint32_t, __builtin_convertvector(f32x2{a, b}, bf16x2));
 }
@@ -368,16 +370,18 @@ __device__ __forceinline__ void mat_tok_body(const MatArgs& a, int bx, int by, u
                         float v0 = xv[xb][t][i][2 * e], v1 = xv[xb][t][i][2 * e + 1];
 #pragma unroll
                         for (int k = 0; k < NS; k++) {
+                            if (NS == 3 && k == 0) {
+                                // three parts: the first cut off, not rounded (which takes the largest finite values
+                                // to infinity); an infinity is its first part, as fp32 products would have it
+                                const uint32_t b0 = __float_as_uint(v0), b1 = __float_as_uint(v1);
+                                part[k][e] = __builtin_amdgcn_perm(b1, b0, 0x07060302u);
+                                v0 = __builtin_fabsf(v0) == __builtin_inff() ? 0.f : v0 - __uint_as_float(b0 & 0xFFFF0000u);
+                                v1 = __builtin_fabsf(v1) == __builtin_inff() ? 0.f : v1 - __uint_as_float(b1 & 0xFFFF0000u);
+                                continue;
+                            }
                             const uint32_t w = pk_bf16(v0, v1);
                             part[k][e] = w;
-                            if (NS == 3 && k == 0) {
-                                // three parts: an infinity is its first part (as fp32 products would have it)
-                                const float h0 = __uint_as_float(w << 16), h1 = __uint_as_float(w & 0xFFFF0000u);
-                                v0 = __builtin_fabsf(h0) == __builtin_inff() ? 0.f : v0 - h0;
-                                v1 = __builtin_fabsf(h1) == __builtin_inff() ? 0.f : v1 - h1;
-                            } else if (k + 1 < NS) {
-                                v0 = rest_bf16<0>(w, v0), v1 = rest_bf16<1>(w, v1);
-                            }
+                            if (k + 1 < NS) v0 = rest_bf16<0>(w, v0), v1 = rest_bf16<1>(w, v1);
                         }
                     }
 #pragma unroll
@@ -399,11 +403,13 @@ __device__ __forceinline__ void mat_tok_body(const MatArgs& a, int bx, int by, u
                     for (int t = 0; t < TT; t++) {
                         f32x4 d[R];
 #pragma unroll
-                        for (int k = 0; k < NS; k++) {
+                        for (int i = 0; i < NS; i++) {
+                            // (three parts from the last: the first two of a value near the largest may sum to 2^128)
+                            const int k = NS == 3 ? NS - 1 - i : i;
                             const bf16x8 part = *reinterpret_cast<const bf16x8*>(L.x[t][k] + xld);
 #pragma unroll
                             for (int r = 0; r < R; r++)
-                                d[r] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(part, wv[r], k ? d[r] : f32x4{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
+                                d[r] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(part, wv[r], i ? d[r] : f32x4{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
                         }
 #pragma unroll
                         for (int r = 0; r < R; r++) {

@@ -359,6 +359,34 @@ def test_token_tile_infinities(qw, n):
     ctx.close()
 
 
+@pytest.mark.parametrize("n", [2, 3, 4, 7, 12, 15])
+def test_token_tile_largest_values(qw, n):
+    """The largest finite inputs below 16 tokens keep their value (a bf16 rounding of them would be infinite). Weights
+    of -1, 0 and 1 and one large value a row and sign keep the fp32 sums finite; the other terms round away, so an
+    output is one fp32 product and its scaling, 2^-23 of it, beside the sum's cancelled terms (2^-24 each)."""
+    rows, cols = 40, 96
+    r = np.random.default_rng(120 + n)
+    w8 = r.integers(-1, 2, (rows, cols)).astype(np.int8)
+    s = (1e-3 * (0.5 + r.random((rows, cols // 32)))).astype(np.float32)
+    x = r.standard_normal((n, cols)).astype(np.float32)
+    # from the least value that bf16 rounds to infinity up to the largest of 22 bits (2^128 - 2^106: beyond it a sum in
+    # another order may itself round past the largest fp32)
+    bigs = np.array([2.0 ** 128 - 2.0 ** 119, 3.4e38, 2.0 ** 128 - 2.0 ** 113, 2.0 ** 128 - 2.0 ** 106]).astype(np.float32)
+    for t in range(n):
+        x[t, (11 * t + 5) % cols] = (-1) ** (t // 4) * bigs[t % 4]
+    ctx = _ctx(qw)
+    y, y2 = torch.zeros((n, rows), device=DEV), torch.zeros((n, rows), device=DEV)
+    ctx.mat(dev(x), y, dev(w8), dev(s))
+    ctx.mat_multi(dev(x), [(y2, dev(w8), dev(s))])
+    torch.cuda.synchronize()
+    want = x.astype(np.float64) @ (w8 * np.repeat(s.astype(np.float64), 32, axis=1)).T
+    mag = np.abs(x.astype(np.float64)) @ np.abs(w8 * np.repeat(s.astype(np.float64), 32, axis=1)).T
+    got = y.cpu().numpy().astype(np.float64)
+    assert np.all(np.isfinite(got)) and np.all(np.abs(got - want) <= 4e-7 * mag)
+    assert torch.equal(y, y2)
+    ctx.close()
+
+
 @pytest.mark.parametrize("n", [3, 20])
 def test_mat_wide_row_stride(qw, oracle, n):
     """Token rows too far apart for the token-tile kernel's offsets go to the other kernels."""
