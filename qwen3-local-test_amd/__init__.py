@@ -135,15 +135,16 @@ def _ptr(t):
     return None if t is None else t.data_ptr()
 
 
-_raw_stream = torch._C._cuda_getCurrentRawStream
-_cuda_device = torch._C._cuda_getDevice
+# (None in a torch without GPU support, where the host helpers here still work)
+_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+_cuda_device = getattr(torch._C, "_cuda_getDevice", None)
 
 
 def _stream(stream):
     """The handle of `stream`, or of the current device's current stream."""
     if stream is not None:
         return stream.cuda_stream
-    if torch.cuda.is_initialized():
+    if _raw_stream and _cuda_device and torch.cuda.is_initialized():
         return _raw_stream(_cuda_device())
     return torch.cuda.current_stream().cuda_stream
 

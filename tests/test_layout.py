@@ -7,6 +7,10 @@ element (position p, KV head h, dim d) where the kernels address it:
   V     = part + (((d/16)*4 + kb/8)*16 + d%16)*8 + kb%8
 k_rows/v_rows must invert them.
 """
+import os
+import subprocess
+import sys
+
 import numpy as np
 import pytest
 
@@ -58,3 +62,25 @@ def test_head_region_is_contiguous_and_grows_by_prefix():
     big_v = qw.v_block(rows).view(nkv, cap2 * D)
     for h in range(nkv):
         assert torch.equal(big_v[h, :cap * D], small_v[h])
+
+
+def test_host_helpers_without_gpu_bindings():
+    """The package loads, and its layout helpers work, in a torch without GPU support (whose _C lacks the CUDA names);
+    the stream handle comes from the public interface where only those names are missing."""
+    code = """
+import sys, torch
+sys.path.insert(0, sys.argv[1])
+for name in ("_cuda_getCurrentRawStream", "_cuda_getDevice"):
+    if hasattr(torch._C, name):
+        delattr(torch._C, name)
+import common
+qw = common.load_package()
+rows = torch.randn(64, 2, 64).half()
+assert torch.equal(qw.k_rows(qw.k_block(rows), 64, 2, 64), rows)
+torch.cuda.is_initialized = lambda: True
+torch.cuda.current_stream = lambda: type("Stream", (), {"cuda_stream": 77})
+assert qw._stream(None) == 77
+"""
+    tests = os.path.dirname(os.path.abspath(__file__))
+    r = subprocess.run([sys.executable, "-c", code, tests], capture_output=True, text=True)
+    assert r.returncode == 0, r.stderr
