@@ -835,6 +835,8 @@ constexpr size_t gemm_lds() {
 
 namespace {
 
+constexpr int kTokGroups = 65535;  // token groups a launch
+
 template <int TT, int R, int NS, int B, int KW>
 hipError_t launch_tok(MatMultiArgs a, hipStream_t s) {
     constexpr size_t lds = tok_lds<TT, R, NS, B, KW>();
@@ -842,8 +844,16 @@ hipError_t launch_tok(MatMultiArgs a, hipStream_t s) {
     if (const hipError_t e = raise_lds((const void*)k_mat_tok<TT, R, NS, B, KW>, lds, raised); e != hipSuccess) return e;
     int wg = 0;
     for (int i = 0; i < a.count; i++) a.wg_end[i] = wg += (a.m[i].rows + 16 * R - 1) / (16 * R);
-    hipLaunchKernelGGL((k_mat_tok<TT, R, NS, B, KW>), dim3(wg, (a.m[0].n + 16 * TT - 1) / (16 * TT)), dim3(64 * KW), lds, s, a);
-    return hipGetLastError();
+    // as many launches as the grid's y limit asks for
+    const int n = a.m[0].n, most = kTokGroups * 16 * TT;
+    for (int t0 = 0;;) {
+        const int nt = std::min(most, n - t0);
+        for (int i = 0; i < a.count; i++) a.m[i].n = nt;
+        hipLaunchKernelGGL((k_mat_tok<TT, R, NS, B, KW>), dim3(wg, (nt + 16 * TT - 1) / (16 * TT)), dim3(64 * KW), lds, s, a);
+        if (const hipError_t e = hipGetLastError(); e != hipSuccess || n - t0 == nt) return e;
+        t0 += nt;
+        for (int i = 0; i < a.count; i++) a.m[i].x += (size_t)nt * a.m[i].x_stride, a.m[i].y += (size_t)nt * a.m[i].y_stride;
+    }
 }
 
 // The token-tile kernel's shapes with two parts a token value. Eight waves (a workgroup a CU) up to 64 tokens, or

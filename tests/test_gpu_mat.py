@@ -387,6 +387,25 @@ def test_token_tile_largest_values(qw, n):
     ctx.close()
 
 
+def test_more_tokens_than_a_grid(qw):
+    """More token groups than a grid's y dimension takes (65,535 of 32 tokens): every token's row. An output is 32
+    products of x split in two, 2^-18 of each left, in one block's sum."""
+    rows, cols, n = 40, 32, 65535 * 32 + 2000
+    g = torch.Generator(device=DEV)
+    g.manual_seed(5)
+    x = torch.randn((n, cols), device=DEV, generator=g)
+    w = torch.randint(-127, 128, (rows, cols), dtype=torch.int8, device=DEV, generator=g)
+    s = 1e-3 * (0.5 + torch.rand((rows, 1), device=DEV, generator=g))
+    y, y2 = (torch.full((n, rows), float("nan"), device=DEV) for _ in range(2))
+    ctx = _ctx(qw)
+    ctx.mat(x, y, w, s)
+    ctx.mat_multi(x, [(y2, w, s)])
+    wd = w.double() * s.double()
+    err = (y.double() - x.double() @ wd.T).abs() / (x.double().abs() @ wd.abs().T)
+    assert float(err.max()) <= 1e-5 and torch.equal(y, y2)  # (a NaN fails either)
+    ctx.close()
+
+
 @pytest.mark.parametrize("n", [3, 20])
 def test_mat_wide_row_stride(qw, oracle, n):
     """Token rows too far apart for the token-tile kernel's offsets go to the other kernels."""
