@@ -123,6 +123,7 @@ struct PrefillArgs {
     int kb_words;
     int list;             // filled by launch_prefill
 };
+constexpr int kPfListMin = 4;       // QSA prefill: a query tile with no more 64-key tiles reads them all
 constexpr int kPfListTiles = 4096;  // QSA prefill: 64-key tiles whose visible ones are listed in LDS, at most
 // Rope widths the prefill kernel's in-kernel query normalization handles: the rotate-half partner of a
 // lane's dim is then in the same lane.

@@ -40,7 +40,10 @@
 //    sees (one pass over the tokens' bits, a ballot per 512 tiles), and walks the list instead of the keys; the
 //    schedule's halves are halves of the listed tiles. 512 tokens on 16,384 keys, blocks of 64, a budget of
 //    2,048 keys (32 of 256 blocks a token, half of a block's score shared by the chunk): 226 -> 151 us. Every
-//    score is masked by its bit as before, so the result does not depend on what the list leaves out.
+//    score is masked by its bit as before, so the result does not depend on what the list leaves out. A query tile
+//    of four key tiles or fewer reads them all, and one that sees all of its tiles walks them without the list; there
+//    the list costs what making it takes, 1.5-2 us (all visible, without / with lists: 64 tokens on 2,000 keys 47.5 /
+//    49.1 us, 2,048 on 32,768 1,105 / 1,117).
 #include "common.hpp"
 #include "kernels.hpp"
 
@@ -745,7 +748,9 @@ __device__ __forceinline__ void pf_segment(const PrefillArgs& a, int kvh, int qt
 
 // QSA: the key tiles of [0, nt) that some token of query tile qt sees, in order, into list[0, count), count >= 1 (an
 // unseen tile stands in where every key is hidden), then three entries nt (past the keys). Returns count. Called by
-// the whole workgroup before any copy; `cnt` holds 8 words.
+// the whole workgroup before any copy; `cnt` holds 8 words. The count, read from LDS, is made a scalar: as a vector
+// value it takes the tile loop's counter and every copy's address along (17 more vector instructions a tile and a lane
+// read per copy: 2,048 tokens on 32,768 keys, all visible, 1,158 -> 1,097 us).
 __device__ __forceinline__ int pf_visible(const PrefillArgs& a, int tok_per_blk, int qt, int nt, uint16_t* list, int* cnt) {
     const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
     const int t0 = qt * tok_per_blk, t1 = min(a.n, t0 + tok_per_blk);
@@ -771,7 +776,7 @@ __device__ __forceinline__ int pf_visible(const PrefillArgs& a, int tok_per_blk,
         __syncthreads();
     }
     if (tid == 0 && count == 0) list[0] = 0;
-    count = max(1, count);
+    count = __builtin_amdgcn_readfirstlane(max(1, count));
     if (tid < 3) list[count + tid] = (uint16_t)nt;
     __syncthreads();
     return count;
@@ -794,27 +799,29 @@ __global__ __launch_bounds__(64 * kPfWaves, 1) void k_prefill(PrefillArgs a) {
     // QSA: tile counts are of the visible tiles, listed in LDS (unless the keys have more tiles than a list holds)
     extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
     int* cnt = reinterpret_cast<int*>(smem + 4 * PfCfg<D>::TILEE * 2 + D * sizeof(float));
-    uint16_t* list0 = reinterpret_cast<uint16_t*>(cnt + kPfWaves);
-    uint16_t* list1 = list0 + a.list;
+    uint16_t* l0 = reinterpret_cast<uint16_t*>(cnt + kPfWaves);
+    uint16_t* l1 = l0 + a.list;
     const bool listed = QSA && a.list > 0;
-    auto tiles = [&](int qt, uint16_t* list) {
+    // (no list where every tile is seen, and none of few tiles)
+    auto tiles = [&](int qt, uint16_t*& list) {
         const int nt = pf_tiles(a, tok_per_blk, qt);
-        return listed ? pf_visible(a, tok_per_blk, qt, nt, list, cnt) : nt;
+        const int seen = listed && nt > kPfListMin ? pf_visible(a, tok_per_blk, qt, nt, list, cnt) : nt;
+        if (seen == nt) list = nullptr;
+        return seen;
     };
-    const uint16_t *l0 = listed ? list0 : nullptr, *l1 = listed ? list1 : nullptr;
     if constexpr (SPLIT) {  // longest tiles first, an equal run of key tiles each
         const int lg = __builtin_ctz((unsigned)a.split_all);
         const int qt = n_qt - 1 - (j >> lg), part = a.split_all - 1 - (j & (a.split_all - 1));
-        const int nt = tiles(qt, list0);
+        const int nt = tiles(qt, l0);
         const PfPart pt = pf_part(nt, a.split_all, part);
         if (part >= pt.parts) return;
         q0 = qt, own0 = part, parts0 = pt.parts, lo0 = pt.lo, hi0 = pt.hi;
         slot0 = parts0 > 1 ? kvh * a.slots + qt : -1;
     } else if (j >= 2 * np) {  // the middle tile
-        q0 = np, lo0 = 0, hi0 = tiles(np, list0), slot0 = -1;
+        q0 = np, lo0 = 0, hi0 = tiles(np, l0), slot0 = -1;
     } else {
         const int p = j >> 1, ql = n_qt - 1 - p;
-        const int nl = tiles(ql, list0), ns = tiles(p, list1);
+        const int nl = tiles(ql, l0), ns = tiles(p, l1);
         const int x = max(0, nl - (nl + ns + 1) / 2);
         slot0 = x > 0 ? kvh * a.slots + p : -1;
         if ((j & 1) == 0) {
@@ -849,7 +856,7 @@ static hipError_t launch_pf_d(const PrefillArgs& a0, int q_dtype, int in_dtype, 
     // entries of a visible-tile list: every key tile and the three after the last; none past what LDS holds
     // beside the tiles (a context of more than 262,144 keys: every tile is read)
     const int nt = (a.pos + a.n + PF_KT - 1) / PF_KT;
-    a.list = a.kbits && nt <= kPfListTiles ? (nt + 4) & ~1 : 0;
+    a.list = a.kbits && nt > kPfListMin && nt <= kPfListTiles ? (nt + 4) & ~1 : 0;
     const int G = a.NH / a.NKV;
     const int tok = PF_ROWS / G;
     const int n_qt = (a.n + tok - 1) / tok;

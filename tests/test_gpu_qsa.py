@@ -465,6 +465,19 @@ def test_prefill_qsa_sparse_tiles(qw, oracle, pos, n, dt, cr, density):
     test_prefill_qsa_parity(qw, oracle, QWEN3_NEXT, pos, n, dt, cr, density, "prefill")
 
 
+# Query tiles (16 tokens) that see every key tile (walked without a list) or have four or fewer, beside ones that see a
+# few of more (walked by a list), in both schedules: the two segments of a paired workgroup differ in it
+@pytest.mark.parametrize("pos,n,dt", [(0, 2100, "bf16"), (0, 2100, "f32"), (200, 100, "f32"), (150, 110, "bf16")])
+def test_prefill_qsa_lists_beside_whole_ranges(qw, oracle, monkeypatch, pos, n, dt):
+    draw = _rand_mask
+
+    def mask(seed, pos, n, cr, density):
+        whole = (np.arange(n) // 16 % 3 == 0)[:, None]
+        return np.where(whole, draw(seed, pos, n, cr, 1.0), draw(seed, pos, n, cr, density))
+    monkeypatch.setitem(globals(), "_rand_mask", mask)
+    test_prefill_qsa_parity(qw, oracle, QWEN3_NEXT, pos, n, dt, 64, 0.05, "prefill")
+
+
 # Query tiles (16 tokens) that see unequal numbers of 64-key tiles, below and above the launch's parts (16, 8 and 4),
 # on two KV heads, so that tiles with few parts lie between tiles with many in the partials' workspace
 @pytest.mark.parametrize("dt", ["f32", "bf16"])
