@@ -214,10 +214,25 @@ struct QsaSelectArgs {
     int hcopies;          // histogram copies a token (n * hcopies <= kQsaHistTokens)
 };
 hipError_t launch_qsa_select(const QsaSelectArgs& a, int in_dtype, hipStream_t s);
-// The same for many tokens (from kQsaMany; at most 32,768 complete blocks; raw, cnt, hist and cand unused): scores
+// The same for many tokens (qsa_many; at most 32,768 complete blocks; raw, cnt, hist and cand unused): scores
 // in one launch, the selections in another.
 hipError_t launch_qsa_select_many(const QsaSelectArgs& a, int in_dtype, hipStream_t s);
-constexpr int kQsaMany = 16, kQsaManyBlocks = 32768;
+constexpr int kQsaManyBlocks = 32768;
+// Heads that the many-token score kernel norms and rotates at once (a pass over its keys each)
+constexpr int qsa_score_heads(int ID) { return ID <= 64 ? 8 : ID <= 128 ? 4 : 2; }
+// Whether a select call takes the many-token launches. The few-token kernel runs a workgroup per 64 blocks of a token,
+// 21 ns each over the chip (a sixteenth for a token that selects nothing); the many-token launches take 14 us and
+// 12.5 more a pass over the heads, or 4 us where no token selects. Whole calls, few / many: 128 dims, 4 heads, 16
+// tokens of 4,100 blocks (1,040 workgroups) 31 / 28 us, 512 of 4,224 634 / 67; 8 heads, the same 16 34 / 40 and 28 of
+// them (1,820) 49 / 40; 16 heads 39 / 65, and 40 of 4,106 (2,600) 80 / 65; 64 heads, 60 of 4,111 (3,900) 243 / 217; 49
+// of 100 tokens selecting from 525 blocks 24 / 29; none of 600 (1,800) 5.8 / 4.9, none of 1,024 (1,024) 4.5 / 5.4.
+inline bool qsa_many(int pos, int n, int cr, int budget, int IH, int ID) {
+    const int nmax = (pos + n) / cr;
+    const long long first = ((long long)budget / cr + 1) * cr - 1;  // the first position that selects
+    const long long sel = first <= pos ? n : first < (long long)pos + n ? pos + n - first : 0;
+    const long long wgs = (nmax + 63) / 64, passes = (IH + qsa_score_heads(ID) - 1) / qsa_score_heads(ID);
+    return n >= 16 && nmax <= kQsaManyBlocks && sel * wgs + (n - sel) * wgs / 16 >= (sel ? 500 + 220 * passes : 96);
+}
 // First-digit histograms (2,048 bins) a select launch may use: a token takes 1 to 8 copies
 constexpr int kQsaHistTokens = 1024;
 // The two-launch form (more than 32,768 complete blocks): selection workgroups of kQsaSelBlocks blocks, each

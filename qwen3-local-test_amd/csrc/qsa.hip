@@ -927,7 +927,6 @@ __global__ __launch_bounds__(kQsaThreads) __attribute__((amdgpu_waves_per_eu(4, 
 // loaded one at a time. The whole index call there 634 -> 62 us: the few-token kernel normed the query again for
 // every 64 blocks and ran the products on vector units, 16 lanes a key.
 constexpr int kQsaTok = 32, kQsaScoreBlocks = 128;
-constexpr int qsa_score_heads(int ID) { return ID <= 64 ? 8 : ID <= 128 ? 4 : 2; }
 template <int IN_DT, int ID>
 __global__ __launch_bounds__(256) void k_qsa_score(QsaSelectArgs a) {
     constexpr int HC = qsa_score_heads(ID), ST = ID + 4, DL = ID / 16;  // heads in LDS, row stride, dims a lane

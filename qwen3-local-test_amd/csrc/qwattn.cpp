@@ -937,14 +937,6 @@ int qwattn_qsa_pool(qwattn_ctx* c, void* stream, const void* ik, int in_dtype, c
     return QWATTN_OK;
 }
 
-// Whether a select call of n tokens, nmax complete blocks for the last, takes the many-token launches: where the
-// few-token kernel would have 3.5 workgroups (64 blocks of a token) a CU or more. Whole calls, few / many: 16 tokens
-// of 4,100 blocks (1,040 workgroups) 34 / 30 us, 12 of them (780) 29 / 29, 100 of 524 (900) 38 / 31, 16 of 64 blocks
-// (16) 12 / 27, 512 of 4,224 634 / 67.
-static bool qsa_many(int n, int nmax) {
-    return n >= qw::kQsaMany && nmax <= qw::kQsaManyBlocks && (long long)n * ((nmax + 63) / 64) >= 896;
-}
-
 int qwattn_qsa_select(qwattn_ctx* c, void* stream, const void* iq, int in_dtype, const float* q_gamma, int idx_heads,
                       int idx_dim, int cr, int budget, const float* pooled, int pos, int n, uint32_t* mask,
                       int mask_words, uint32_t* key_bits, int kb_words) {
@@ -974,7 +966,7 @@ int qwattn_qsa_select(qwattn_ctx* c, void* stream, const void* iq, int in_dtype,
     if (int rc = take_wait_error(c)) return rc;
     DeviceGuard dg(c->device);
     const int stride = (std::max(1, nmax) + 3) & ~3;  // score rows padded to whole 16-byte loads
-    const bool many = qsa_many(n, nmax);
+    const bool many = qw::qsa_many(pos, n, cr, budget, idx_heads, idx_dim);
     const int per = (int)std::min<size_t>(many ? n : std::min(c->qsa_hist_n, qw::qsa_select_tokens(nmax)),
                                           std::max<size_t>(1, kQsaScoreBytes / ((size_t)stride * sizeof(float))));
     for (int t0 = 0; t0 < n; t0 += per) {
@@ -1003,7 +995,7 @@ int qwattn_qsa_index(qwattn_ctx* c, void* stream, const void* ik, const void* iq
     const int stride = (std::max(1, nmax) + 3) & ~3;  // score rows padded to whole 16-byte loads
     const int per = (int)std::min<size_t>(std::min(c->qsa_hist_n, qw::qsa_select_tokens(nmax)),
                                           std::max<size_t>(1, kQsaScoreBytes / ((size_t)stride * sizeof(float))));
-    if (cr < 2 || nmax != pos / cr || n > per || qsa_many(n, nmax)) {
+    if (cr < 2 || nmax != pos / cr || n > per || qw::qsa_many(pos, n, cr, budget, idx_heads, idx_dim)) {
         // a block completes (or the tokens take several select launches): the pooling launch, then the select
         if (int rc = qwattn_qsa_pool(c, stream, ik, in_dtype, k_gamma, idx_dim, cr, raw, pooled, cap, pos, n)) return rc;
         return qwattn_qsa_select(c, stream, iq, in_dtype, q_gamma, idx_heads, idx_dim, cr, budget, pooled, pos, n,
