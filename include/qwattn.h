@@ -307,10 +307,10 @@ int qwattn_qsa_index(qwattn_ctx* ctx, void* stream, const void* ik, const void* 
 
 /* The projections either side of the attention layer: Qwen4Vulkan::mat (src/qwen4_vk.cpp:848-856) on its
  * matrix-vector pipelines q4_matmul_q8 / q4_matmul_f32 (shaders/q4_matmul.comp, codecs C_Q8 / C_F32 of
- * shaders/q4_codec.glsl) and, from 16 tokens, its tiled GEMM pipelines q4_gemm_q8 / q4_gemm_f32
- * (shaders/q4_gemm.comp; here on MFMA with fp32-level accuracy: a skinny kernel for Q8 up to 64 tokens and
- * for Q8 matrices of up to 1,024 rows, a tiled GEMM otherwise). y[t][r] (row stride y_stride) = sum_c W[r][c] x[t][c] (row stride x_stride) for
- * t < n, r < rows, with W planar Q8_0 when q8 != 0 (w: int8 [rows][cols], s: float [rows][cols/32], one
+ * shaders/q4_codec.glsl) and its tiled GEMM pipelines q4_gemm_q8 / q4_gemm_f32 (shaders/q4_gemm.comp; here on
+ * MFMA with fp32-level accuracy: Q8 from two tokens on a token-tile kernel, or on a tiled GEMM where its tiles
+ * take less, from 65 tokens at the earliest; fp32 weights from 16 on a tiled GEMM). y[t][r] (row stride
+ * y_stride) = sum_c W[r][c] x[t][c] (row stride x_stride) for t < n, r < rows, with W planar Q8_0 when q8 != 0 (w: int8 [rows][cols], s: float [rows][cols/32], one
  * scale per 32 consecutive weights of a row, as qwattn_q8_unpack writes them) or float [rows][cols] (s
  * unused); post 1 then applies y = silu(y * post_scale) (the shader's `post`). fp32 arithmetic. cols a
  * multiple of 32 (q8) or 16 (f32); x_stride >= cols and a multiple of 4; y_stride >= rows; w and x 16-byte
@@ -332,9 +332,9 @@ typedef struct qwattn_mat_out {
 /* count (1..4) projections of the same input x in one call, with the results of count qwattn_mat calls.
  * No counterpart in the reference, which issues one Qwen4Vulkan::mat per matrix (the query, key and value
  * projections of a full-attention layer: src/qwen4_vk.cpp:965-967); for callers that project one input
- * several ways: below 16 tokens one matrix-vector launch streams every matrix (one launch's latency
- * instead of count), from 16 tokens each matrix runs as its own qwattn_mat call. All matrices share cols, q8, x,
- * x_stride and n; each is checked as qwattn_mat checks it. */
+ * several ways: one launch streams every matrix (one launch's latency instead of count), except those that a
+ * tiled GEMM takes (Q8 from 65 tokens at the earliest, fp32 from 16), which run as their own qwattn_mat calls.
+ * All matrices share cols, q8, x, x_stride and n; each is checked as qwattn_mat checks it. */
 int qwattn_mat_multi(qwattn_ctx* ctx, void* stream, const qwattn_mat_out* mats, int count, int q8, int cols,
                      const float* x, int x_stride, int n);
 

@@ -88,7 +88,7 @@ public:
               "qwattn_mat");
     }
 
-    // count projections of one input (qwattn_mat_multi: one launch below 16 tokens).
+    // count projections of one input (qwattn_mat_multi: one launch but for the tiled GEMMs).
     void mat_multi(void* stream, const qwattn_mat_out* mats, int count, bool q8, int cols, const float* x, int x_stride,
                    int n) {
         check(ctx_, qwattn_mat_multi(ctx_, stream, mats, count, q8 ? 1 : 0, cols, x, x_stride, n), "qwattn_mat_multi");

@@ -929,7 +929,7 @@ hipError_t launch_gemm_q8(const MatArgs& a, hipStream_t s) {
 }
 
 // The Q8 GEMM's tiles with what a 64-column step of one takes a CU, in hundredths of a microsecond (one tile a CU;
-// 2,048 tokens through 8,192 x 2,048 and 2,048 x 4,096: 147 / 183 / 216 and 109 / 85 / 103 us).
+// 2,048 tokens through 8,192 x 2,048 and 2,048 x 4,096: 147 / 184 / 213 and 107 / 86 / 107 us).
 struct GemmTile {
     int bm, bn, step;
     hipError_t (*launch)(const MatArgs&, hipStream_t);
@@ -952,9 +952,13 @@ bool gemm_fits(const MatArgs& a) { return gemm_offsets_fit(a.cols, a.x_stride); 
 
 // Whether a Q8 matrix takes the token-tile kernel (from two tokens on): up to 64 tokens, else where its 64-row x
 // 32-token workgroups, two a CU and 0.55 us a pair and 64 columns, take less than the GEMM's tiles (8,192 x 2,048
-// at 128 / 256 / 512 tokens 29 / 37 / 68 us against 29 / 31 / 48; 2,048 x 4,096 at 256 / 512 / 777 20 / 36 / 64
-// against 50 / 51 / 53; 512 x 2,048 at 2,048 26 against 28). By the matrix alone, so that qwattn_mat and
-// qwattn_mat_multi agree.
+// at 128 / 256 / 512 tokens 21 / 37 / 68 us against 29 / 31 / 46; 2,048 x 4,096 at 256 / 512 / 777 22 / 39 / 66
+// against 50 / 51 / 52; 512 x 2,048 at 2,048 27 against 29). By the matrix alone, so that qwattn_mat and
+// qwattn_mat_multi agree. For the same reason a small matrix called by itself with 2 to 15 tokens stays here although a
+// matrix-vector kernel of fp32 multiply-adds is faster then (256 x 2,048 at 4 / 8 / 15 tokens 5.2 / 6.2 / 7.2 us, 4.6 /
+// 4.7 / 4.7): beside a larger one in qwattn_mat_multi it costs this kernel next to nothing, but on matrix-vector
+// workgroups in the same launch 8,192 + 512 + 512 rows of 2,048 columns went from 11.4 / 11.9 us at 4 / 8 tokens to
+// 12.6 / 15.1.
 bool tok_wins(const MatArgs& a) {
     if (a.n <= 64) return true;
     const long long wgs = (long long)((a.rows + 63) / 64) * ((a.n + 31) / 32);

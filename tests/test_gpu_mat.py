@@ -95,11 +95,10 @@ def test_mat_rejects_bad_shapes(qw):
     ctx.close()
 
 
-# The MFMA kernels from 16 tokens (columns a multiple of 32). Q8 up to 64 tokens, Q8 matrices of up to 1,024
-# rows at any token count, and Q8 launches the GEMM would cut into fewer than 256 tiles: the skinny kernel with 16, 32 or 64 tokens a workgroup (partial row and
-# token groups, waves with no column blocks at 96 columns); otherwise, and fp32 weights: the tiled GEMM with
-# each token tile width (128 when that still gives 512 workgroups, else 64 when that does, else 32). The
-# attention layer's shapes among them.
+# The MFMA kernels from 16 tokens (columns a multiple of 32). Q8: the token-tile kernel to a few hundred tokens (partial
+# row and token groups, waves with no columns at 96 of them) and the tiled GEMM where its tiles take less; fp32
+# weights: the fp32 GEMM with each token tile width (128 when that still gives 512 workgroups, else 64 when that does,
+# else 32). The attention layer's shapes among them.
 GEMM_CASES = [(512, 2048, 16), (512, 2048, 200), (100, 96, 33), (37, 1056, 130), (2048, 4096, 64),
               (8192, 2048, 20), (300, 64, 257), (160, 256, 1100), (64, 64, 1500),
               (8192, 64, 512), (8000, 96, 530), (8192, 64, 1100), (8000, 96, 1030),
@@ -139,7 +138,7 @@ def test_gemm_f32_parity(qw, oracle, rows, cols, n):
 
 @pytest.mark.parametrize("n", [40, 200])
 def test_gemm_strides_post_and_scale_range(qw, oracle, n):
-    """The MFMA kernels (skinny at 40 tokens, tiled at 200) with x_stride / y_stride wider than the rows,
+    """The token-tile kernel (eight waves at 40 tokens, four at 200) with x_stride / y_stride wider than the rows,
     post 1, outputs beyond `rows` untouched, and inputs whose magnitudes span 2^-20 .. 2^20 (the hi / lo
     split keeps fp32 range and relative accuracy)."""
     rows, cols = 200, 512
@@ -184,8 +183,8 @@ def test_gemm_full_prefill_matches_matvec(qw):
 
 @pytest.mark.parametrize("n", [1, 4, 5, 40])
 def test_mat_multi_equals_separate_calls(qw, oracle, n):
-    """qwattn_mat_multi (one matrix-vector launch over several matrices below 16 tokens, one GEMM a matrix
-    from 16) gives each matrix the bits of its own qwattn_mat call, and the oracle's values: the attention
+    """qwattn_mat_multi (one matrix-vector launch over several matrices of one token, one token-tile launch of more, a
+    launch a matrix that the GEMM takes) gives each matrix the bits of its own qwattn_mat call, and the oracle's values: the attention
     layer's query + gate, key and value projections of one input (8,192 + 512 + 512 rows, one row a wave
     below 4,096 rows in total, four from there), then three small ones."""
     print(f"mat_multi n={n}", flush=True)
