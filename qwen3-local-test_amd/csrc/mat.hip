@@ -216,8 +216,8 @@ __device__ __forceinline__ void split_bf16(const float (&v)[8], bf16x8& hi, bf16
 // What bounds it is the rate of the vector-memory pipe and of instruction issue, not HBM. A load costs one cycle
 // per 64-byte piece it touches, so an operand loaded straight in the MFMA layout (lane l: row l % 16) costs 64
 // cycles a kilobyte; loaded by consecutive lanes it costs 16, and a pass through the wave's own part of the LDS
-// (written as loaded, read as operands, both free of bank conflicts by the XORs below; in-order within the
-// wave) gives the layout. 9,216 x 2,048 at 4 / 77 tokens, one box: 10.9 / 31.1 us with operand-layout loads,
+// (written as loaded, read as operands, spread over the banks by the XORs below: conflicts are 0.4 of its active
+// cycles, and waves wait for it 6% of theirs at 77 tokens; in-order within the wave) gives the layout. 9,216 x 2,048 at 4 / 77 tokens, one box: 10.9 / 31.1 us with operand-layout loads,
 // 8.5 / 20.7 us through the LDS; the kernels before (fp32 multiply-adds on up to 4 tokens a workgroup; 32-row
 // workgroups with operand-layout loads from 16) took 16.0 / 86 us. A vector instruction, the conversions
 // included, takes a SIMD 2.0-2.5 ns.
@@ -683,8 +683,9 @@ __global__ __launch_bounds__(512, RT * TT == 1 ? 4 : 2) void k_gemm_q8(MatArgs a
         xv[i] = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(
             rx, (int)gemm_x_off(32 * i + (tid >> 4), xq, k, a.x_stride, nkb), 0, 0));
     };
-    // LDS rows of 64 columns are eight 16-byte chunks, chunk q of row r at q ^ (r / 2) % 8: operand reads (16
-    // rows' chunk q) and the loaders' writes are free of bank conflicts
+    // LDS rows of 64 columns are eight 16-byte chunks, chunk q of row r at q ^ (r / 2) % 8, which spreads operand reads
+    // (16 rows' chunk q) and the loaders' writes over the banks: conflicts are 0.17 of the LDS's active cycles (256 x
+    // 128 tiles), and waves wait for it 5% of theirs
     auto at = [](int r, int q) { return r * 128 + ((q ^ ((r >> 1) & 7)) << 4); };
     // the conversion of the loaded pieces in units of a few instructions: four to each half of a weight piece (its
     // pairs of weights), two to a token piece

@@ -919,8 +919,8 @@ __global__ __launch_bounds__(kQsaThreads) __attribute__((amdgpu_waves_per_eu(4, 
 // Scores of 32 tokens x 128 blocks a workgroup (four waves, 32 blocks each): sum over the heads of
 // relu(q_h . pooled), each product a chain of v_mfma_f32_32x32x2_f32 (fp32 multiply-adds, as the 16-lane dot
 // products of the few-token kernel). A lane (c, h) holds block c's dims [h ID/2, + ID/2) in registers; the tokens'
-// heads are normed and rotated once a workgroup into LDS (rows padded by 16 bytes: their 16-byte reads are free
-// of bank conflicts), 512 head dims at a time. Stored as the few-token kernel stores them: ~score
+// heads are normed and rotated once a workgroup into LDS (rows padded by 16 bytes, which spreads their
+// 16-byte reads over the banks: waves wait for the LDS under 1% of their cycles), 512 head dims at a time. Stored as the few-token kernel stores them: ~score
 // for a token's complete blocks, 0 past them (to the row's end). A token that selects nothing is left out.
 // Bound: the fp32 matrix rate (2.2 GFLOP take 14 us of the chip at 153 TFLOP/s, a large product here), in whole
 // 32 x 32 tiles a wave: 512 tokens x 4,224 blocks of 4 heads x 128 dims (2.06 tiles a SIMD) 43 us; 53 with the rows

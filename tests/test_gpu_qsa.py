@@ -102,7 +102,7 @@ CASES = {
 TIE_PERIOD = {"ties_cr8": 37, "ties_cr4_8k": 37, "ties_cr2_64k": 101, "ties_long_cr2": 1009}  # blocks
 
 
-# Calls that score on the matrix cores (16 tokens and more, 896 workgroups of 64 blocks): every indexer width, heads
+# Calls that score on the matrix cores (16 tokens and more, of enough blocks for their heads): every indexer width, heads
 # in one and several groups, dense tokens beside selecting ones, partial token groups, 8, 16 and 32 keys a selecting
 # thread, exact ties
 MANY = {
